@@ -1,0 +1,43 @@
+"""The matrix prefill's GEMM tiles, splits of K and row kernels at the sizes where they can go wrong:
+prompts just past and short of tile edges (64, 128, 256 rows), FFN widths of an odd number of 32s (the
+32-wide K steps) and of less than a tile of columns, and products that split K up to 8 ways.
+
+Against the oracle's full causal block, over a stack of 2 layers: layer 1's K and V rows depend on all
+of layer 0.  Bars: layer 0's rows within 1 bf16 ulp of the oracle's in 99.9% of elements; layer 1's
+with an RMS difference of at most 2^-7 of their RMS.  A bf16 rounding moves a value by up to 2^-9 of
+it; about 8 of them lie between the embedding and layer 1's rows, independent ones add to
+sqrt(8) 2^-9 = 0.0055.  A wrong tile, row or part of a sum moves the rows by their own size."""
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_prefill import bf16_ulps, build, kv_rows, oracle_kv_and_logits
+from tiles_amd import runtime as R
+from tiles_amd.tileplan import package as K
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hidden,intermediate,heads,kv_heads,length,std", [
+    (256, 544, 4, 1, 66, 0.08),       # 65 rows; down projection over 544 = 17 x 32
+    (128, 32, 2, 1, 129, 0.12),       # 128 rows; gate/up and down narrower than any tile
+    (256, 512, 4, 2, 130, 0.08),      # 129 rows
+    (512, 1056, 8, 2, 257, 0.05),     # 256 rows; 33 x 32
+    (2048, 8192, 32, 8, 71, 0.02),    # 64-row tiles, K split up to 8 ways
+    (2048, 8192, 32, 8, 514, 0.02),   # 128-row tiles, K split
+])
+def test_matrix_prefill_at_tile_edges(tmp_path, hidden, intermediate, heads, kv_heads, length, std):
+    spec, path, packed, ospec = build(tmp_path, hidden, intermediate, heads, kv_heads, 2, 512, 640, seed=7 + length, std=std)
+    prompt = np.random.default_rng(length).integers(0, 512, length).tolist()
+    ctx = R.DecoderModel(R.load_plan(path)).create_context()
+    snapshot = ctx.collect(ctx.enqueue_prefill(prompt, kv=True))["kv"]
+    got = kv_rows(snapshot, K.read_plan(path), 2, length, kv_heads * 64)
+    want, _ = oracle_kv_and_logits(prompt, packed, ospec, 2, kv_heads * 64)
+    for i, name in enumerate("KV"):
+        ulps = bf16_ulps(got[0][i], want[0][i])
+        assert float((ulps <= 1).mean()) >= 0.999, name
+        rms = lambda a: float(np.sqrt((a.astype(np.float64) ** 2).mean()))  # noqa: E731
+        off = rms(got[1][i] - want[1][i]) / rms(want[1][i])
+        print(f"{hidden}/{intermediate}, {length} tokens, {name}: layer 0 equal {float((ulps == 0).mean()):.4f}, "
+              f"layer 1 off by {off:.5f} of its RMS", flush=True)
+        assert off <= 2.0 ** -7, name

@@ -6,17 +6,19 @@
 // writes are the ones a position-by-position prefill writes, up to the FP32 summation order of
 // the dot products:
 //
-//   u = bf16(bf16(x * rsqrt(mean(x^2) + eps)) * attn_norm)      rms_rows
-//   q, k, v = bf16(W u)                                          gemm_bf16 (MFMA, FP32 sums)
+//   u = bf16(bf16(x * rsqrt(mean(x^2) + eps)) * attn_norm)      norm_rows
+//   q, k, v = bf16(W u)                                          GEMM (MFMA, FP32 sums)
 //   q, k rotated as the worker rotates them; K, V rows -> cache  rope_rows
 //   s = bf16(bf16(q . k) * (1 / sqrt(dh)));                       attention_tiles (causal: M the
 //   P = bf16(exp(s - M) / S); attention = bf16(sum P v)          row's maximum, S its FP32 exp-sum)
-//   r = bf16(bf16(Wo attention) + x)                             GEMM, add_rows
-//   z = RMSNorm(r) with ffn_norm                                 rms_rows
-//   p = bf16(bf16(silu(bf16(Wgate z))) * bf16(Wup z))            GEMMs, silu_rows
-//   y = bf16(bf16(Wdown p) + r)                                  GEMM, add_rows
+//   r = bf16(bf16(Wo attention) + x)                             GEMM with the residual
+//   z = RMSNorm(r) with ffn_norm                                 norm_rows
+//   p = bf16(bf16(silu(bf16(Wgate z))) * bf16(Wup z))            one GEMM over both matrices
+//   y = bf16(bf16(Wdown p) + r)                                  GEMM with the residual
 //
-// The GEMMs are this file's MFMA kernel rather than a library's: rocBLAS, linked into this
+// A GEMM too small for the chip splits K; the kernel after it adds the parts (norm_rows, rope_rows).
+//
+// The GEMMs are this library's MFMA kernel rather than a library's: rocBLAS, linked into this
 // library, conflicted with the different rocBLAS build PyTorch ships, and a process that loaded
 // this library before importing torch crashed.
 #include "prefill.hpp"
@@ -26,6 +28,7 @@
 #include <string>
 
 #include "device_common.hpp"
+#include "prefill_gemm.hpp"
 #include "worker_config.hpp"
 
 namespace tiles {
@@ -38,76 +41,162 @@ constexpr int kTile = 64;  // key positions per attention tile
 __device__ inline float bf(uint16_t bits) { return bf16_bits_to_float(bits); }
 __device__ inline uint16_t bits16(float v) { return static_cast<uint16_t>(float_to_bf16_bits(v)); }
 
-// Sum over the block's threads (kRowThreads), in a fixed order.
-__device__ float block_sum(float v, float* partial)
+// The rows a GEMM left: bf16 rows (splits 1), or the FP32 sums of its parts of K, `plane` elements
+// apart.
+struct GemmRows {
+    const uint16_t* rows;
+    const float* partial;
+    int splits;
+    size_t plane;
+};
+
+// Eight adjacent values of a GEMM's rows from element `at`, rounded to bf16.  The number of parts is
+// a template argument so that their loads are in flight together.
+template <int kSplits>
+__device__ inline void load_rows8(const GemmRows& g, size_t at, float (&v)[8])
 {
-    for (int offset = 32; offset > 0; offset >>= 1)
-        v += __shfl_xor(v, offset);
-    if ((threadIdx.x & 63) == 0)
-        partial[threadIdx.x / 64] = v;
-    __syncthreads();
-    float total = 0.0f;
-    for (int w = 0; w < kRowThreads / 64; ++w)
-        total += partial[w];
-    __syncthreads();
-    return total;
+    if constexpr (kSplits == 1) {
+        const u32x4 bits = *reinterpret_cast<const u32x4*>(g.rows + at);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            v[e] = Bf::elem(bits, e);
+    } else {
+        f32x4 part[kSplits][2];
+#pragma unroll
+        for (int p = 0; p < kSplits; ++p) {
+            const f32x4* from = reinterpret_cast<const f32x4*>(g.partial + p * g.plane + at);
+            part[p][0] = from[0];
+            part[p][1] = from[1];
+        }
+#pragma unroll
+        for (int p = 1; p < kSplits; ++p) {
+            part[0][0] += part[p][0];
+            part[0][1] += part[p][1];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            v[e] = Bf::round(part[0][e / 4][e % 4]);
+    }
 }
 
-// x[r] = the embedding row of tokens[r].
+constexpr int kMostSplits = 8;
+// f(std::integral_constant<int, splits>{}).
+template <int kSplits = 1, typename F>
+void with_splits(int splits, const F& f)
+{
+    if (splits == kSplits)
+        f(std::integral_constant<int, kSplits>{});
+    else if constexpr (kSplits < kMostSplits)
+        with_splits<kSplits + 1>(splits, f);
+}
+
+// x[r] = the embedding row of tokens[r], 16 bytes a thread.
 __global__ void __launch_bounds__(kRowThreads) gather_rows(const uint16_t* embedding, const ti_token_id* tokens, int d,
                                                            uint16_t* x)
 {
-    const uint16_t* src = embedding + static_cast<size_t>(tokens[blockIdx.x]) * d;
-    uint16_t* dst = x + static_cast<size_t>(blockIdx.x) * d;
-    for (int i = threadIdx.x; i < d; i += kRowThreads)
+    const u32x4* src = reinterpret_cast<const u32x4*>(embedding + static_cast<size_t>(tokens[blockIdx.x]) * d);
+    u32x4* dst = reinterpret_cast<u32x4*>(x + static_cast<size_t>(blockIdx.x) * d);
+    for (int i = threadIdx.x; i < d / 8; i += kRowThreads)
         dst[i] = src[i];
 }
 
-// out[r] = bf16(bf16(x[r] * inv_rms) * scale), inv_rms = 1 / sqrt(mean(x[r]^2) + eps) in FP32,
-// as the worker's rms_apply computes it.
-__global__ void __launch_bounds__(kRowThreads) rms_rows(const uint16_t* x, const uint16_t* scale, int d, float eps,
-                                                        uint16_t* out)
+// out[r] = bf16(bf16(x[r] * inv_rms) * scale), inv_rms = 1 / sqrt(mean(x[r]^2) + eps) in FP32, as the
+// worker's rms_apply computes it.  Of a GEMM that left parts (kSplits > 1), x[r] is
+// bf16(bf16(sum) + residual[r]) and also goes to sum_out.  One block a row, 16 bytes a load, the row
+// in registers between its two passes: at 4,096 rows of 2,048 from memory 8.6 us (2 bytes a load,
+// the row read twice: 14.3), at 36 rows the latency of its loads.
+template <int kSplits>
+__global__ void __launch_bounds__(kRowThreads) norm_rows(GemmRows sums, const uint16_t* x, const uint16_t* scale, int d, float eps,
+                                                         uint16_t* sum_out, uint16_t* out)
 {
+    constexpr int kMost = kMaxHidden / 8 / kRowThreads;  // 16-byte vectors of a row a thread holds
     __shared__ float partial[kRowThreads / 64];
-    const uint16_t* row = x + static_cast<size_t>(blockIdx.x) * d;
+    const size_t first = static_cast<size_t>(blockIdx.x) * d;
+    float v[kMost][8];
     float squares = 0.0f;
-    for (int i = threadIdx.x; i < d; i += kRowThreads) {
-        const float v = bf(row[i]);
-        squares = fmaf(v, v, squares);
+#pragma unroll
+    for (int i = 0; i < kMost; ++i) {
+        const int n = (i * kRowThreads + threadIdx.x) * 8;
+        if (n < d) {
+            const u32x4 bits = *reinterpret_cast<const u32x4*>(x + first + n);
+            float sum[8];
+            if constexpr (kSplits > 1)
+                load_rows8<kSplits>(sums, first + n, sum);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[i][e] = kSplits > 1 ? Bf::round(sum[e] + Bf::elem(bits, e)) : Bf::elem(bits, e);
+                squares = fmaf(v[i][e], v[i][e], squares);
+            }
+            if constexpr (kSplits > 1)
+                *reinterpret_cast<u32x4*>(sum_out + first + n) = pack_bf16(v[i]);
+        }
     }
-    const float total = block_sum(squares, partial);
+    const float wave_sum = group_sum<64>(squares);
+    if ((threadIdx.x & 63) == 63)
+        partial[threadIdx.x / 64] = wave_sum;
+    __syncthreads();
+    float total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kRowThreads / 64; ++w)
+        total += partial[w];
     const float inv = 1.0f / sqrtf(total / static_cast<float>(d) + eps);
-    uint16_t* dst = out + static_cast<size_t>(blockIdx.x) * d;
-    for (int i = threadIdx.x; i < d; i += kRowThreads)
-        dst[i] = bits16(Bf::round(Bf::round(bf(row[i]) * inv) * bf(scale[i])));
+#pragma unroll
+    for (int i = 0; i < kMost; ++i) {
+        const int n = (i * kRowThreads + threadIdx.x) * 8;
+        if (n < d) {
+            const u32x4 bits = *reinterpret_cast<const u32x4*>(scale + n);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[i][e] = Bf::round(v[i][e] * inv) * Bf::elem(bits, e);
+            *reinterpret_cast<u32x4*>(out + first + n) = pack_bf16(v[i]);
+        }
+    }
 }
 
-// Row r of qkv ([q heads | k heads | v heads], bf16) at position `position + r`: the query and
-// key heads rotated (split halves; cos and sin of position * frequency rounded to bf16, each
-// product rounded, then the difference or sum), the query heads to q_rot, the key and value
-// heads to the cache row of the position.
-__global__ void __launch_bounds__(kRowThreads) rope_rows(const uint16_t* qkv, int position, const float* frequencies, int nq,
-                                                         int nkv, int dh, uint16_t* q_rot, uint16_t* key_cache,
-                                                         uint16_t* value_cache)
+// Row r of the Q/K/V product ([q heads | k heads | v heads]; nq 0: [k heads | v heads]) at position
+// `position + r`: the query and key heads rotated (split halves; cos and sin of position * frequency
+// rounded to bf16, each product rounded, then the difference or sum), the query heads to q_rot, the
+// key and value heads to the cache row of the position.  A block computes its position's cos and sin
+// once and rotates 8 pairs a thread: 13.3 us for 4,096 rows of 40 heads (20.1 with cos and sin computed
+// for every pair and 2 bytes a load).
+template <int DH, int kSplits>
+__global__ void __launch_bounds__(kRowThreads) rope_rows(GemmRows qkv, int position, const float* frequencies, int nq, int nkv,
+                                                         uint16_t* q_rot, uint16_t* key_cache, uint16_t* value_cache)
 {
-    const int r = blockIdx.x;
-    const int pos = position + r;
-    const int half = dh / 2;
-    const uint16_t* src = qkv + static_cast<size_t>(r) * (nq + 2 * nkv) * dh;
-    for (int index = threadIdx.x; index < (nq + nkv) * half; index += kRowThreads) {
-        const int head = index / half, pair = index - head * half;
-        const float angle = static_cast<float>(pos) * frequencies[pair];
-        const float c = Bf::round(cosf(angle)), s = Bf::round(sinf(angle));
-        const float a = bf(src[head * dh + pair]), b = bf(src[head * dh + pair + half]);
-        const uint16_t lo = bits16(Bf::round(Bf::round(a * c) - Bf::round(b * s)));
-        const uint16_t hi = bits16(Bf::round(Bf::round(b * c) + Bf::round(a * s)));
-        uint16_t* dst = head < nq ? q_rot + (static_cast<size_t>(r) * nq + head) * dh
-                                  : key_cache + (static_cast<size_t>(pos) * nkv + head - nq) * dh;
-        dst[pair] = lo;
-        dst[pair + half] = hi;
+    constexpr int kHalf = DH / 2, kVectors = kHalf / 8;
+    __shared__ float cosine[kHalf], sine[kHalf];
+    const int r = blockIdx.x, pos = position + r;
+    const size_t first = static_cast<size_t>(r) * (nq + 2 * nkv) * DH;
+    if (threadIdx.x < kHalf) {
+        const float angle = static_cast<float>(pos) * frequencies[threadIdx.x];
+        cosine[threadIdx.x] = Bf::round(cosf(angle));
+        sine[threadIdx.x] = Bf::round(sinf(angle));
     }
-    for (int index = threadIdx.x; index < nkv * dh; index += kRowThreads)
-        value_cache[static_cast<size_t>(pos) * nkv * dh + index] = src[(nq + nkv) * dh + index];
+    __syncthreads();
+    const int rotated = (nq + nkv) * kVectors, all = rotated + nkv * DH / 8;
+    for (int index = threadIdx.x; index < all; index += kRowThreads) {
+        if (index >= rotated) {
+            const int at = (index - rotated) * 8;
+            float v[8];
+            load_rows8<kSplits>(qkv, first + (nq + nkv) * DH + at, v);
+            *reinterpret_cast<u32x4*>(value_cache + static_cast<size_t>(pos) * nkv * DH + at) = pack_bf16(v);
+            continue;
+        }
+        const int head = index / kVectors, pair = (index - head * kVectors) * 8;
+        float a[8], b[8], lo[8], hi[8];
+        load_rows8<kSplits>(qkv, first + head * DH + pair, a);
+        load_rows8<kSplits>(qkv, first + head * DH + pair + kHalf, b);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float c = cosine[pair + e], s = sine[pair + e];
+            lo[e] = Bf::round(a[e] * c) - Bf::round(b[e] * s);
+            hi[e] = Bf::round(b[e] * c) + Bf::round(a[e] * s);
+        }
+        uint16_t* dst = head < nq ? q_rot + (static_cast<size_t>(r) * nq + head) * DH
+                                  : key_cache + (static_cast<size_t>(pos) * nkv + head - nq) * DH;
+        *reinterpret_cast<u32x4*>(dst + pair) = pack_bf16(lo);
+        *reinterpret_cast<u32x4*>(dst + pair + kHalf) = pack_bf16(hi);
+    }
 }
 
 // Causal attention on the matrix cores, for 64 rows (positions position + r0 ..) and every
@@ -377,129 +466,74 @@ attention_tiles(const uint16_t* q_rot, int position, int rows, int nq, int nkv,
         }
 }
 
-// out = bf16(a + b) elementwise (a and b bf16).
-__global__ void __launch_bounds__(kRowThreads) add_rows(const uint16_t* a, const uint16_t* b, size_t count, uint16_t* out)
-{
-    for (size_t i = blockIdx.x * static_cast<size_t>(kRowThreads) + threadIdx.x; i < count;
-         i += static_cast<size_t>(gridDim.x) * kRowThreads)
-        out[i] = bits16(Bf::round(bf(a[i]) + bf(b[i])));
-}
+// The tile shapes of the GEMM, and the time in us a 64-wide K step of one takes a CU that runs one
+// block of it, and two at a time (measured at Llama-3.2-1B's widths, 36 to 4,096 rows).  The largest
+// tile reads the least from L2 per product and wins where its blocks fill the chip; the smaller ones
+// fill it with fewer rows and, at 64 rows, stream W at 3.9 TB/s where it is read once.
+struct TileShape {
+    int bm, bn;
+    float alone, paired;  // paired 0: two do not fit a CU's LDS
+};
+constexpr TileShape kTileShapes[] = {{256, 256, 2.03f, 0.0f}, {128, 128, 0.85f, 1.1f}, {128, 64, 0.52f, 0.74f}, {64, 64, 0.29f, 0.46f}};
+constexpr float kBlockStart = 2.4f;         // us a block takes besides its K steps
+constexpr float kPartialRate = 3.1e6f;      // bytes per us that partial sums are written and read back at
+constexpr int kCus = 256;
+constexpr size_t kPartialFloats = 16u << 20;  // 64 MiB of partial sums
 
-// out = bf16(bf16(silu(gate)) * up), silu(g) = g / (1 + exp(-g)) in FP32 (gate and up bf16).
-__global__ void __launch_bounds__(kRowThreads) silu_rows(const uint16_t* gate, const uint16_t* up, size_t count, uint16_t* out)
-{
-    for (size_t i = blockIdx.x * static_cast<size_t>(kRowThreads) + threadIdx.x; i < count;
-         i += static_cast<size_t>(gridDim.x) * kRowThreads) {
-        const float g = bf(gate[i]);
-        out[i] = bits16(Bf::round(Bf::round(g / (1.0f + expf(-g))) * bf(up[i])));
-    }
-}
+struct Tiling {
+    int shape, splits;
+};
 
-// C = A B^T (kBRows: B is [N][K], a weight matrix whose rows are output features) or C = A B
-// (!kBRows: B is [K][N], Wdown as stored), all bf16 and row-major, A [M][K]; C rounded to bf16
-// from FP32 sums (ldc: C's row stride).  Tiles of 128 x 128 per block of 4 waves, each wave
-// 64 x 64 as 4 x 4 v_mfma_f32_16x16x32_bf16 tiles, K in steps of 32 through LDS (rows padded to
-// 40 elements: 16-byte operand reads of 16 rows 80 bytes apart fall on distinct bank groups; a
-// [K][N] B tile stays as loaded and its operands come from gfx950's transposing LDS reads), the
-// next step's tile loaded into registers while this one's MFMAs run.  K % 32 == 0 and N % 16 == 0
-// (the launcher checks); rows and columns past M and N are clamped on load and not stored.
-constexpr int kGemmTile = 128, kGemmK = 32, kGemmStride = kGemmK + 8;
-
-template <bool kBRows>
-__global__ void __launch_bounds__(256) gemm_bf16(const uint16_t* a, const uint16_t* b, uint16_t* c, int m, int n, int k, int ldc)
+// The tile shape and split of K with the least estimated time: blocks of a CU run one after another,
+// or in pairs.  The estimate picks within 2% of the fastest measured choice on average over nine row
+// counts from 36 to 4,096 and the four products of a Llama-3.2-1B layer (13% at worst).
+Tiling choose_tiling(int m, int columns, int k, bool may_split)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t as[kGemmTile * kGemmStride];
-    // kBRows: B as [n][k] rows; !kBRows: B as loaded, [k][n] rows kBkStride apart, its operands
-    // read by transposing LDS reads.
-    __shared__ __attribute__((aligned(16))) uint16_t bs[kGemmTile * kGemmStride];
-    constexpr int kBkStride = kGemmTile + 16;  // 288-byte rows: four rows of a transposing read on distinct banks
-    static_assert(kGemmK * kBkStride <= kGemmTile * kGemmStride, "B tile exceeds its LDS area");
-    const int t = threadIdx.x, lane = t & 63, wave = t / 64;
-    const int m0 = blockIdx.y * kGemmTile, n0 = blockIdx.x * kGemmTile;
-    const int wm = (wave / 2) * 64, wn = (wave % 2) * 64;
-    // Loads of one K step: A rows t / 2 (16 elements each half), B likewise (kBRows) or B rows
-    // k = t / 8 of 16 columns each (!kBRows).
-    const int arow = min(m0 + t / 2, m - 1), acol = (t % 2) * 16;
-    const int brow = kBRows ? min(n0 + t / 2, n - 1) : t / 8;
-    const int bcol = kBRows ? (t % 2) * 16 : min(n0 + (t % 8) * 16, n - 16);
-    u32x4 ra[2], rb[2];
-    auto load = [&](int k0) {
-        const u32x4* pa = reinterpret_cast<const u32x4*>(a + static_cast<size_t>(arow) * k + k0 + acol);
-        ra[0] = pa[0];
-        ra[1] = pa[1];
-        const u32x4* pb = kBRows ? reinterpret_cast<const u32x4*>(b + static_cast<size_t>(brow) * k + k0 + bcol)
-                                 : reinterpret_cast<const u32x4*>(b + static_cast<size_t>(k0 + brow) * n + bcol);
-        rb[0] = pb[0];
-        rb[1] = pb[1];
-    };
-    auto store = [&]() {
-        u32x4* da = reinterpret_cast<u32x4*>(as + (t / 2) * kGemmStride + acol);
-        da[0] = ra[0];
-        da[1] = ra[1];
-        if constexpr (kBRows) {
-            u32x4* db = reinterpret_cast<u32x4*>(bs + (t / 2) * kGemmStride + bcol);
-            db[0] = rb[0];
-            db[1] = rb[1];
-        } else {
-            u32x4* db = reinterpret_cast<u32x4*>(bs + brow * kBkStride + (t % 8) * 16);
-            db[0] = rb[0];
-            db[1] = rb[1];
-        }
-    };
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int r = lane % 16, q = (lane / 16) * 8;
-    load(0);
-    for (int k0 = 0; k0 < k; k0 += kGemmK) {
-        __syncthreads();  // the previous step's operand reads are done
-        store();
-        __syncthreads();
-        if (k0 + kGemmK < k)
-            load(k0 + kGemmK);
-        u32x4 fa[4], fb[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            fa[i] = *reinterpret_cast<const u32x4*>(as + (wm + i * 16 + r) * kGemmStride + q);
-            if constexpr (kBRows) {
-                fb[i] = *reinterpret_cast<const u32x4*>(bs + (wn + i * 16 + r) * kGemmStride + q);
-            } else {
-                // ds_read_b64_tr_b16: within a 16-lane group, lane j names row q + 4 h + j / 4,
-                // columns wn + 16 i + 4 (j % 4) .. + 3, and lane r receives column wn + 16 i + r
-                // of the group's four rows.
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    typedef short v4s __attribute__((ext_vector_type(4)));
-                    const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (__attribute__((address_space(3))) v4s*)(bs + (q + 4 * h + (r >> 2)) * kBkStride + wn + i * 16 + 4 * (r & 3)));
-                    const uint2 pair = __builtin_bit_cast(uint2, v);
-                    fb[i][2 * h] = pair.x;
-                    fb[i][2 * h + 1] = pair.y;
-                }
+    Tiling best{0, 1};
+    float least = INFINITY;
+    const int steps = k / 64;
+    for (int shape = 0; shape < 4; ++shape) {
+        const TileShape& t = kTileShapes[shape];
+        const long tiles = static_cast<long>((m + t.bm - 1) / t.bm) * ((columns + t.bn - 1) / t.bn);
+        for (int splits = 1; splits <= (may_split ? kMostSplits : 1); ++splits) {
+            if (splits > 1 && (steps / splits < 4 || static_cast<size_t>(splits) * m * columns > kPartialFloats))
+                break;
+            const long per_cu = (tiles * splits + kCus - 1) / kCus;
+            const int part = (steps + splits - 1) / splits;
+            float time = t.paired > 0.0f ? (per_cu / 2) * (part * t.paired + kBlockStart) + (per_cu % 2) * (part * t.alone + kBlockStart)
+                                         : per_cu * (part * t.alone + kBlockStart);
+            if (splits > 1)
+                time += static_cast<float>(splits) * m * columns * sizeof(float) / kPartialRate;
+            if (time < least) {
+                least = time;
+                best = {shape, splits};
             }
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                acc[i][j] = mfma_16x16x32_bf16(fa[i], fb[j], acc[i][j]);
     }
-    // Lane l holds rows 4 (l / 16) .. + 3 of column l % 16 of each 16 x 16 tile.
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int col = n0 + wn + j * 16 + r;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = m0 + wm + i * 16 + (lane / 16) * 4 + e;
-                if (row < m && col < n)
-                    c[static_cast<size_t>(row) * ldc + col] = bits16(Bf::round(acc[i][j][e]));
-            }
-        }
+    return best;
+}
+
+template <int BM, int BN, int WM, int WN, int KS, int STAGES, GemmOut OUT>
+void launch_gemm(hipStream_t stream, GemmArgs g)
+{
+    const int columns = OUT == GemmOut::kSilu ? 2 * g.n : g.n;
+    g.m_tiles = (g.m + BM - 1) / BM;
+    g.n_tiles = (columns + BN - 1) / BN;
+    hipLaunchKernelGGL((gemm_tiles<BM, BN, WM, WN, KS, STAGES, OUT>), dim3(g.m_tiles * g.n_tiles * g.splits),
+                       dim3((BM / WM) * (BN / WN) * 64), 0, stream, g);
+}
+
+template <GemmOut OUT>
+void launch_shape(hipStream_t stream, int shape, const GemmArgs& g)
+{
+    // kSilu groups four MFMA tiles of columns, so its waves take 64.
+    constexpr bool kWide = OUT == GemmOut::kSilu;
+    switch (shape) {
+    case 0: return launch_gemm<256, 256, 128, 64, 64, 2, OUT>(stream, g);
+    case 1: return launch_gemm<128, 128, kWide ? 32 : 64, kWide ? 64 : 32, 64, 2, OUT>(stream, g);
+    case 2: return launch_gemm<128, 64, kWide ? 32 : 64, kWide ? 64 : 32, 64, 3, OUT>(stream, g);
+    default: return launch_gemm<64, 64, kWide ? 16 : 32, kWide ? 64 : 32, 64, 4, OUT>(stream, g);
+    }
 }
 
 } // namespace
@@ -512,9 +546,9 @@ bool MatrixPrefill::supports(const ti_worker_program_view& p)
         s.query_heads % s.kv_heads != 0 || s.query_heads / s.kv_heads > kMaxGroup)
         return false;
     // Every GEMM of MatrixPrefill::layer, as (K, N): Q/K/V (d, heads x dh), Wo (query width, d),
-    // gate/up (d, f), down (f, d).  gemm() takes K a multiple of kGemmK and N a multiple of 16; the
+    // gate/up (d, f), down (f, d).  The GEMM takes K a multiple of 32 and N a multiple of 16; the
     // head widths are multiples of 64 already.  A stack outside these prefills through the worker.
-    auto gemm_shape = [](int k, int n) { return k >= kGemmK && k % kGemmK == 0 && n >= 16 && n % 16 == 0; };
+    auto gemm_shape = [](int k, int n) { return k >= 32 && k % 32 == 0 && n >= 16 && n % 16 == 0; };
     const int d = s.hidden_size, f = s.intermediate_size, qw = s.query_heads * dh, kvw = s.kv_heads * dh;
     return gemm_shape(d, qw) && gemm_shape(d, kvw) && gemm_shape(qw, d) && gemm_shape(d, f) && gemm_shape(f, d);
 }
@@ -529,48 +563,62 @@ MatrixPrefill::~MatrixPrefill()
 
 namespace {
 struct Views {
-    uint16_t *x, *u, *qkv, *q, *attention, *projected, *r, *gate, *up;
+    uint16_t *x, *u, *qkv, *q, *attention, *r, *product;
+    float* partial;
 };
 size_t row_elements(const ti_model_shape& s)
 {
     const size_t d = s.hidden_size, f = s.intermediate_size;
     const size_t qkv = static_cast<size_t>(s.query_heads + 2 * s.kv_heads) * s.head_dim;
     const size_t q = static_cast<size_t>(s.query_heads) * s.head_dim;
-    return 5 * d + qkv + q + 2 * f;  // x, u, attention, projected, r | qkv | q | gate, up
+    return 3 * d + qkv + 2 * q + f;  // x, u, r | qkv | q, attention | product
 }
 Views views(void* buffer, const ti_model_shape& s, size_t rows)
 {
-    const size_t d = s.hidden_size, f = s.intermediate_size;
-    uint16_t* at = static_cast<uint16_t*>(buffer);
-    auto take = [&](size_t per_row) {
-        uint16_t* v = at;
-        at += rows * per_row;
-        return v;
-    };
+    const size_t d = s.hidden_size, q = static_cast<size_t>(s.query_heads) * s.head_dim;
     Views v{};
+    v.partial = static_cast<float*>(buffer);
+    uint16_t* at = reinterpret_cast<uint16_t*>(v.partial + kPartialFloats);
+    auto take = [&](size_t per_row) {
+        uint16_t* start = at;
+        at += rows * per_row;
+        return start;
+    };
     v.x = take(d);
     v.u = take(d);
-    v.attention = take(d);
-    v.projected = take(d);
     v.r = take(d);
     v.qkv = take(static_cast<size_t>(s.query_heads + 2 * s.kv_heads) * s.head_dim);
-    v.q = take(static_cast<size_t>(s.query_heads) * s.head_dim);
-    v.gate = take(f);
-    v.up = take(f);
+    v.q = take(q);
+    v.attention = take(q);
+    v.product = take(s.intermediate_size);
     return v;
 }
 
-// C (rows x n, row stride ldc) = X (rows x k) W^T, W (n x k) row-major; or = X W with W (k x n).
-int gemm(hipStream_t stream, bool w_rows, const uint16_t* x, int rows, int k, const uint16_t* w, int n, uint16_t* c, int ldc)
+// Enqueues X W^T of x [m][k] and w [n][k] into rows of c, or as partial sums; returns where the
+// product is.  With a residual (row stride n), c receives bf16(bf16(sum) + residual) unless the
+// sums are partial: the kernel that adds those adds the residual too.
+GemmRows gemm(hipStream_t stream, const uint16_t* x, int m, int k, const uint16_t* w, int n, const uint16_t* residual, uint16_t* c,
+              int ldc, float* partial)
 {
-    if (rows < 1 || k % kGemmK != 0 || n % 16 != 0 || n < 16 || ldc < n)
-        return fail(TI_ERR_INVALID_ARGUMENT, "prefill GEMM shape (K a multiple of 32, N of 16)");
-    const dim3 grid((n + kGemmTile - 1) / kGemmTile, (rows + kGemmTile - 1) / kGemmTile);
-    if (w_rows)
-        hipLaunchKernelGGL(gemm_bf16<true>, grid, dim3(256), 0, stream, x, w, c, rows, n, k, ldc);
+    GemmArgs g{x, w, nullptr, residual, c, partial, m, n, k, ldc, 1, 0, 0};
+    if (k % 64 != 0) {  // an FFN width of an odd number of 32s: K in steps of 32
+        if (residual)
+            launch_gemm<128, 128, 64, 32, 32, 3, GemmOut::kResidual>(stream, g);
+        else
+            launch_gemm<128, 128, 64, 32, 32, 3, GemmOut::kRows>(stream, g);
+        return {c, nullptr, 1, 0};
+    }
+    const Tiling t = choose_tiling(m, n, k, partial != nullptr);
+    g.splits = t.splits;
+    if (t.splits > 1) {
+        launch_shape<GemmOut::kPartial>(stream, t.shape, g);
+        return {nullptr, partial, t.splits, static_cast<size_t>(m) * n};
+    }
+    if (residual)
+        launch_shape<GemmOut::kResidual>(stream, t.shape, g);
     else
-        hipLaunchKernelGGL(gemm_bf16<false>, grid, dim3(256), 0, stream, x, w, c, rows, n, k, ldc);
-    return TI_OK;
+        launch_shape<GemmOut::kRows>(stream, t.shape, g);
+    return {c, nullptr, 1, 0};
 }
 } // namespace
 
@@ -578,54 +626,69 @@ int MatrixPrefill::layer(hipStream_t stream, void* kv, int layer, int position, 
 {
     const ti_model_shape& s = p_.shape;
     const int d = s.hidden_size, f = s.intermediate_size, dh = s.head_dim, nq = s.query_heads, nkv = s.kv_heads;
-    const int qw = nq * dh, kvw = nkv * dh, qkvw = qw + 2 * kvw;
+    const int qw = nq * dh, kvw = nkv * dh;
     const Views v = views(buffer_, s, kChunkRows);
-    const uint16_t* base = static_cast<const uint16_t*>(p_.weights) + p_.stack.layer_weights_offset +
-                           static_cast<size_t>(layer) * p_.stack.layer_weight_stride;
     const ti_layer_layout& w = p_.layout;
+    auto weights = [&](int of) {
+        return static_cast<const uint16_t*>(p_.weights) + p_.stack.layer_weights_offset +
+               static_cast<size_t>(of) * p_.stack.layer_weight_stride;
+    };
+    const uint16_t* base = weights(layer);
     uint16_t* cache = static_cast<uint16_t*>(kv) + static_cast<size_t>(layer) * p_.stack.layer_kv_stride;
     const float eps = p_.numeric.rms_norm_eps;
-    const size_t hidden_count = static_cast<size_t>(rows) * d, ffn_count = static_cast<size_t>(rows) * f;
-    const dim3 elementwise(static_cast<unsigned>(std::min<size_t>(4096, (ffn_count + kRowThreads - 1) / kRowThreads)));
-    int code = TI_OK;
-    auto gemm_ok = [&](int status) {
-        code = status;
-        return status == TI_OK;
+    // out = RMSNorm(x), x first completed (into sum_out) by the residual when the GEMM left parts.
+    auto norm = [&](const GemmRows& sums, const uint16_t* residual, uint16_t* sum_out, const uint16_t* scale) {
+        with_splits(sums.splits, [&](auto n) {
+            hipLaunchKernelGGL(norm_rows<n>, dim3(rows), dim3(kRowThreads), 0, stream, sums, n > 1 ? residual : sum_out, scale, d,
+                               eps, sum_out, v.u);
+        });
     };
 
-    hipLaunchKernelGGL(rms_rows, dim3(rows), dim3(kRowThreads), 0, stream, v.x, base + w.attn_norm, d, eps, v.u);
-    // Wq, Wk and Wv are consecutive in the package's layer layout (plan.cpp checks the regions):
-    // one GEMM over their rows, which also fills the chip (Wk and Wv alone are 4 column tiles).
+    if (layer == 0)
+        norm({v.x, nullptr, 1, 0}, nullptr, v.x, base + w.attn_norm);
+    // The prompt's last position goes through the worker, and the positions here are read again only
+    // as cache rows: the last layer ends with its K and V.
+    const bool last = layer + 1 == p_.stack.layers;
+    const int first_row = last ? qw : 0, width = (last ? 0 : qw) + 2 * kvw;
+    GemmRows qkv{v.qkv, nullptr, 1, 0};
+    // Wq, Wk and Wv are consecutive in the package's layer layout (plan.cpp checks the regions): one
+    // GEMM over their rows.
     if (w.Wk == w.Wq + static_cast<uint32_t>(qw) * d && w.Wv == w.Wk + static_cast<uint32_t>(kvw) * d) {
-        if (!gemm_ok(gemm(stream, true, v.u, rows, d, base + w.Wq, qkvw, v.qkv, qkvw)))
-            return code;
-    } else if (!gemm_ok(gemm(stream, true, v.u, rows, d, base + w.Wq, qw, v.qkv, qkvw)) ||
-               !gemm_ok(gemm(stream, true, v.u, rows, d, base + w.Wk, kvw, v.qkv + qw, qkvw)) ||
-               !gemm_ok(gemm(stream, true, v.u, rows, d, base + w.Wv, kvw, v.qkv + qw + kvw, qkvw))) {
-        return code;
+        qkv = gemm(stream, v.u, rows, d, base + w.Wq + static_cast<size_t>(first_row) * d, width, nullptr, v.qkv, width, v.partial);
+    } else {
+        if (!last)
+            gemm(stream, v.u, rows, d, base + w.Wq, qw, nullptr, v.qkv, width, nullptr);
+        gemm(stream, v.u, rows, d, base + w.Wk, kvw, nullptr, v.qkv + width - 2 * kvw, width, nullptr);
+        gemm(stream, v.u, rows, d, base + w.Wv, kvw, nullptr, v.qkv + width - kvw, width, nullptr);
     }
-    hipLaunchKernelGGL(rope_rows, dim3(rows), dim3(kRowThreads), 0, stream, v.qkv, position, p_.rotary_frequencies, nq, nkv, dh,
-                       v.q, cache + w.key, cache + w.value);
-    const float scale = 1.0f / sqrtf(static_cast<float>(dh));
-    const dim3 attention_grid((rows + kAttnRows - 1) / kAttnRows, nkv);
+    const int rotated_queries = last ? 0 : nq;
+    auto rope = [&](auto head_dim) {
+        with_splits(qkv.splits, [&](auto n) {
+            hipLaunchKernelGGL((rope_rows<head_dim, n>), dim3(rows), dim3(kRowThreads), 0, stream, qkv, position,
+                               p_.rotary_frequencies, rotated_queries, nkv, v.q, cache + w.key, cache + w.value);
+        });
+    };
     if (dh == 64)
-        hipLaunchKernelGGL(attention_tiles<64>, attention_grid, dim3(kAttnThreads), 0, stream, v.q, position, rows, nq, nkv,
-                           cache + w.key, cache + w.value, scale, v.attention);
+        rope(std::integral_constant<int, 64>{});
     else
-        hipLaunchKernelGGL(attention_tiles<128>, attention_grid, dim3(kAttnThreads), 0, stream, v.q, position, rows, nq, nkv,
-                           cache + w.key, cache + w.value, scale, v.attention);
-    if (!gemm_ok(gemm(stream, true, v.attention, rows, qw, base + w.Wo, d, v.projected, d)))
-        return code;
-    hipLaunchKernelGGL(add_rows, elementwise, dim3(kRowThreads), 0, stream, v.projected, v.x, hidden_count, v.r);
-    hipLaunchKernelGGL(rms_rows, dim3(rows), dim3(kRowThreads), 0, stream, v.r, base + w.ffn_norm, d, eps, v.u);
-    if (!gemm_ok(gemm(stream, true, v.u, rows, d, base + w.Wgate, f, v.gate, f)) ||
-        !gemm_ok(gemm(stream, true, v.u, rows, d, base + w.Wup, f, v.up, f)))
-        return code;
-    hipLaunchKernelGGL(silu_rows, elementwise, dim3(kRowThreads), 0, stream, v.gate, v.up, ffn_count, v.gate);
-    // Wdown row-major [hidden][intermediate] on the device (ti_relayout_weights).
-    if (!gemm_ok(gemm(stream, true, v.gate, rows, f, base + w.Wdown, d, v.projected, d)))
-        return code;
-    hipLaunchKernelGGL(add_rows, elementwise, dim3(kRowThreads), 0, stream, v.projected, v.r, hidden_count, v.x);
+        rope(std::integral_constant<int, 128>{});
+    if (!last) {
+        const float scale = 1.0f / sqrtf(static_cast<float>(dh));
+        const dim3 attention_grid((rows + kAttnRows - 1) / kAttnRows, nkv);
+        if (dh == 64)
+            hipLaunchKernelGGL(attention_tiles<64>, attention_grid, dim3(kAttnThreads), 0, stream, v.q, position, rows, nq, nkv,
+                               cache + w.key, cache + w.value, scale, v.attention);
+        else
+            hipLaunchKernelGGL(attention_tiles<128>, attention_grid, dim3(kAttnThreads), 0, stream, v.q, position, rows, nq, nkv,
+                               cache + w.key, cache + w.value, scale, v.attention);
+        const GemmRows projected = gemm(stream, v.attention, rows, qw, base + w.Wo, d, v.x, v.r, d, v.partial);
+        norm(projected, v.x, v.r, base + w.ffn_norm);
+        GemmArgs ffn{v.u, base + w.Wgate, base + w.Wup, nullptr, v.product, nullptr, rows, f, d, f, 1, 0, 0};
+        launch_shape<GemmOut::kSilu>(stream, choose_tiling(rows, 2 * f, d, false).shape, ffn);
+        // Wdown row-major [hidden][intermediate] on the device (ti_relayout_weights).
+        const GemmRows down = gemm(stream, v.product, rows, f, base + w.Wdown, d, v.r, v.x, d, v.partial);
+        norm(down, v.r, v.x, weights(layer + 1) + w.attn_norm);
+    }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return hip_fail(e, "prefill kernel launch");
@@ -641,7 +704,7 @@ int MatrixPrefill::enqueue(hipStream_t stream, void* kv, const ti_token_id* toke
     if (position < 0 || position + count > p_.shape.max_context)
         return fail(TI_ERR_INVALID_ARGUMENT, "sequence context capacity reached");
     if (!buffer_) {
-        buffer_bytes_ = row_elements(p_.shape) * kChunkRows * sizeof(uint16_t);
+        buffer_bytes_ = kPartialFloats * sizeof(float) + row_elements(p_.shape) * kChunkRows * sizeof(uint16_t);
         const hipError_t e = hipMalloc(&buffer_, buffer_bytes_);
         if (e != hipSuccess) {
             buffer_ = nullptr;
