@@ -11,11 +11,37 @@ sqrt(8) 2^-9 = 0.0055.  A wrong tile, row or part of a sum moves the rows by the
 import numpy as np
 import pytest
 
-from tests.test_gpu_prefill import bf16_ulps, build, kv_rows, oracle_kv_and_logits
+from oracle import decoder as ref
+from tests.test_gpu_prefill import bf16_ulps, kv_rows, oracle_kv_and_logits
 from tiles_amd import runtime as R
 from tiles_amd.tileplan import package as K
+from tiles_amd.tileplan import plan as P
+from tiles_amd.tileplan import probe
 
 pytestmark = pytest.mark.gpu
+
+
+def check(tmp_path, hidden, intermediate, heads, kv_heads, length, std):
+    dims = dict(hidden_size=hidden, intermediate_size=intermediate, num_attention_heads=heads, num_key_value_heads=kv_heads,
+                head_dim=hidden // heads, max_context=length + 8)
+    spec = P.StackSpec(P.BlockSpec(**dims), 2, 512, True)
+    path = tmp_path / "pkg"
+    K.build_stack_package(spec, K.random_weights(spec, seed=7 + length, std=std), probe.probe_library(), path, "bfloat16")
+    packed = K.read_weights(path, spec, "bfloat16")
+    width = kv_heads * (hidden // heads)
+    prompt = np.random.default_rng(length).integers(0, 512, length).tolist()
+    ctx = R.DecoderModel(R.load_plan(path)).create_context()
+    snapshot = ctx.collect(ctx.enqueue_prefill(prompt, kv=True))["kv"]
+    got = kv_rows(snapshot, K.read_plan(path), 2, length, width)
+    want, _ = oracle_kv_and_logits(prompt, packed, ref.Spec(**dims, layers=2, vocab_size=512), 2, width)
+    for i, name in enumerate("KV"):
+        ulps = bf16_ulps(got[0][i], want[0][i])
+        assert float((ulps <= 1).mean()) >= 0.999, name
+        rms = lambda a: float(np.sqrt((a.astype(np.float64) ** 2).mean()))  # noqa: E731
+        off = rms(got[1][i] - want[1][i]) / rms(want[1][i])
+        print(f"{hidden}/{intermediate}, {length} tokens, {name}: layer 0 equal {float((ulps == 0).mean()):.4f}, "
+              f"layer 1 off by {off:.5f} of its RMS", flush=True)
+        assert off <= 2.0 ** -7, name
 
 
 @pytest.mark.parametrize("hidden,intermediate,heads,kv_heads,length,std", [
@@ -27,17 +53,16 @@ pytestmark = pytest.mark.gpu
     (2048, 8192, 32, 8, 514, 0.02),   # 128-row tiles, K split
 ])
 def test_matrix_prefill_at_tile_edges(tmp_path, hidden, intermediate, heads, kv_heads, length, std):
-    spec, path, packed, ospec = build(tmp_path, hidden, intermediate, heads, kv_heads, 2, 512, 640, seed=7 + length, std=std)
-    prompt = np.random.default_rng(length).integers(0, 512, length).tolist()
-    ctx = R.DecoderModel(R.load_plan(path)).create_context()
-    snapshot = ctx.collect(ctx.enqueue_prefill(prompt, kv=True))["kv"]
-    got = kv_rows(snapshot, K.read_plan(path), 2, length, kv_heads * 64)
-    want, _ = oracle_kv_and_logits(prompt, packed, ospec, 2, kv_heads * 64)
-    for i, name in enumerate("KV"):
-        ulps = bf16_ulps(got[0][i], want[0][i])
-        assert float((ulps <= 1).mean()) >= 0.999, name
-        rms = lambda a: float(np.sqrt((a.astype(np.float64) ** 2).mean()))  # noqa: E731
-        off = rms(got[1][i] - want[1][i]) / rms(want[1][i])
-        print(f"{hidden}/{intermediate}, {length} tokens, {name}: layer 0 equal {float((ulps == 0).mean()):.4f}, "
-              f"layer 1 off by {off:.5f} of its RMS", flush=True)
-        assert off <= 2.0 ** -7, name
+    check(tmp_path, hidden, intermediate, heads, kv_heads, length, std)
+
+
+@pytest.mark.parametrize("hidden,intermediate,heads,kv_heads,length,std", [
+    (1024, 256, 16, 16, 1090, 0.03),  # one query head a K/V head; 2 heads and 32 rows a block
+    (2048, 256, 32, 16, 2120, 0.02),  # two; 4 heads and 64 rows a block, a last block of 7 rows
+    (512, 256, 4, 1, 300, 0.05),      # head_dim 128
+    (1024, 256, 8, 4, 90, 0.03),      # head_dim 128, two query heads a K/V head
+])
+def test_matrix_prefill_attention_forms(tmp_path, hidden, intermediate, heads, kv_heads, length, std):
+    """The attention's heads per wave (as many as leave two blocks a CU), query groups smaller than a
+    wave takes, and both head widths."""
+    check(tmp_path, hidden, intermediate, heads, kv_heads, length, std)

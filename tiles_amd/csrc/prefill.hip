@@ -37,6 +37,7 @@ namespace {
 using Bf = Num<true>;
 constexpr int kRowThreads = 256;
 constexpr int kTile = 64;  // key positions per attention tile
+constexpr int kCus = 256;
 
 __device__ inline float bf(uint16_t bits) { return bf16_bits_to_float(bits); }
 __device__ inline uint16_t bits16(float v) { return static_cast<uint16_t>(float_to_bf16_bits(v)); }
@@ -199,271 +200,273 @@ __global__ void __launch_bounds__(kRowThreads) rope_rows(GemmRows qkv, int posit
     }
 }
 
-// Causal attention on the matrix cores, for 64 rows (positions position + r0 ..) and every
-// query head of K/V head blockIdx.y: wave w takes rows r0 + 16 w .. + 15.  Scores are
-// computed transposed, S^T = K Q^T with v_mfma_f32_16x16x32_bf16 (A: 16 key rows, B: the 16
-// query rows of one head), so that lane l holds query l % 16 against keys 4 (l / 16) + i of each
-// 16-key subtile.  Each score is bf16(bf16(dot) * scale) (the decode worker's score_of), keys past
-// the query's position are masked (tiles past the block's first row only; rows past the chunk
-// compute finite values nobody stores).  Pass 1 keeps each lane's running maximum and exp-sum per
-// head, rescaled when the maximum grows, and merges the four lanes of a query at the end (exact
-// maximum M, FP32 S).  Pass 2 recomputes the scores, rounds P = exp(s - M) / S to bf16 in
-// registers and takes P V on the matrix cores with P as the A operand straight from the score
-// layout: a 32-key step's k-elements 8 g .. 8 g + 7 of lane group g are keys 4 g .. 4 g + 3 and
-// 16 + 4 g .. + 3 of the step (the sum over keys does not depend on their order), and two
-// transposing LDS reads of the V rows supply the same keys.  The block stages each 64-key tile's
-// K rows (and, in pass 2, V rows) in LDS once for its four waves, as stored, while the next
-// tile's rows load into registers.
-// The output is rounded once.  Keys past the block's last position are clamped to it when loaded
-// and masked.
+// Causal attention on the matrix cores: 64-key tiles of one K/V head (blockIdx.y) against 16 HEADS query
+// rows a block.  A wave takes 16 rows (positions position + r0 ..) and HEADS of the group's query heads;
+// waves of a block share its K and V tiles.
+//
+// Scores are computed transposed, S^T = K Q^T with v_mfma_f32_16x16x32_bf16 (A: 16 key rows, B: the 16
+// query rows of one head), so that lane l holds query l % 16 against keys 4 (l / 16) + i of each 16-key
+// subtile.  Each score is bf16(bf16(dot) * scale) (the decode worker's score_of); keys past the query's
+// position are masked (in tiles past the wave's first row only; rows past the chunk compute finite
+// values nobody stores).  Pass 1 keeps each lane's running maximum M and sum S of 2^((s - M) log2 e) per
+// head, rescaled when the maximum grows, and merges the four lanes of a query at the end.  Pass 2
+// recomputes the scores, takes P = exp(s - M) / S as 2^((s - M) log2 e - log2 S), rounds it to bf16 once
+// and multiplies: O^T = V^T P^T with P as the B operand straight from the score layout: a 32-key step's
+// k-elements 8 g .. 8 g + 7 of lane group g are keys 4 g .. 4 g + 3 and 16 + 4 g .. + 3 of the step (the
+// sum over keys does not depend on their order), and two transposing LDS reads of the V rows supply the
+// same keys.  The output is rounded once.
+//
+// What bounds it is the arithmetic per score, once per pass: rounding to bf16 (a conversion for two, an
+// unpacking each), the maximum, one FMA, v_exp_f32, in pass 2 the rounding of P: 7 instructions a score
+// and pass.  The library's exponential and a division per score took 1.7 to 2.1 times as long: 4,096
+// rows of 32 heads at position 0 421 us, now 205-217 (0.33 PFLOP/s), 28,672 rows in seven chunks 17.6 ms
+// a layer, now 7.6; 210 rows, where one wave then took all four heads, 33 us, now 8.  The exponent's
+// rounding moves P by at most a few 2^-23 of it, 2^-13 of the bf16 rounding that follows: layer 1's K
+// and V rows of 130 to 4,000-token prompts are 0.00439-0.00450 and 0.00390-0.00394 off 64 bits either way.
+//
+// K rows (and, in pass 2, V rows) go from memory straight into one of two LDS buffers while the other's
+// tile is used: chunk c (16 bytes) of row r at c ^ r mod 8, the rows of an operand read on distinct
+// banks.  Keys past the block's last position are clamped to it when loaded and masked.
 constexpr int kAttnThreads = 256;
-constexpr int kAttnRows = 64;  // query positions per block: 16 per wave
 
-// Two waves per SIMD for head_dim 64 (256 registers a lane at most; unbounded, the compiler
-// took 276 and ran one); 128 needs more than 256 in either case.
-template <int DH>
+template <int DH, int HEADS>
 __global__ void __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(DH == 64 ? 2 : 1)))
-attention_tiles(const uint16_t* q_rot, int position, int rows, int nq, int nkv,
-                                                                const uint16_t* key_cache, const uint16_t* value_cache,
-                                                                float scale, uint16_t* out)
+attention_tiles(const uint16_t* q_rot, int position, int rows, int nq, int nkv, const uint16_t* key_cache,
+                const uint16_t* value_cache, float scale, uint16_t* out)
 {
+    static_assert(kMaxGroup == 4, "four waves share a group of up to four heads");
+    constexpr int kHeadWaves = kMaxGroup / HEADS;            // waves of a block with the same rows
+    constexpr int kRows = 16 * (kAttnThreads / 64) / kHeadWaves;
     constexpr int KS = DH / 32;                              // 32-dim steps of a score
     constexpr int NT = DH / 16;                              // 16-dim output tiles
-    constexpr int kVStride = DH + 8;                         // bf16 per staged V row
-    constexpr int kKStride = DH + 8;                         // bf16 per staged K row
-    constexpr int kVectors = DH / 8;                         // 16-byte vectors of a K or V row
-    constexpr int kLoads = kTile * kVectors / kAttnThreads;  // vectors per thread per tile
-    static_assert(kTile * kVectors % kAttnThreads == 0, "whole vectors per thread");
-    __shared__ __attribute__((aligned(16))) uint16_t vs[kTile * kVStride];
-    __shared__ __attribute__((aligned(16))) uint16_t ks[kTile * kKStride];
-    // Causal blocks differ in work by their row block (block x reads x + 1 key tiles at position
-    // 0).  Every block is resident at once, two per CU, and the dispatcher gives blocks L and L + H
-    // (H = half the grid) the same CU; launched in row-block order those two were alike, and the
-    // CUs holding two of the last row blocks set the kernel's time.  So block L takes the L-th
-    // heaviest (row block, head) and block L + H the L-th lightest: the two add up to one
-    // average pair.  Any assignment covers every (row block, head) once.
+    constexpr int kVectors = DH / 8;                         // 16-byte chunks of a K or V row
+    constexpr int kRowsPerLoad = 64 / kVectors;              // rows one load of a wave covers
+    constexpr int kLoads = kTile / kRowsPerLoad / (kAttnThreads / 64);
+    constexpr float kLog2e = 1.44269504f;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2][2][kTile * DH];  // buffer, K or V
+    // Causal blocks differ in work by their row block (block x reads x + 1 key tiles at position 0).
+    // With at most two blocks a CU, all are resident at once and the dispatcher gives blocks L and
+    // L + H (H = half the grid) the same CU: block L takes the L-th heaviest (row block, head) and
+    // block L + H the L-th lightest, which add up to one average pair.  A larger grid starts with its
+    // heaviest.  Any assignment covers every (row block, head) once.
     const int row_blocks = gridDim.x, items = gridDim.x * gridDim.y, half = (items + 1) / 2;
     const int linear = blockIdx.x + gridDim.x * blockIdx.y;
-    const int heaviest = linear < half ? linear : items - 1 - (linear - half);  // index in descending weight
+    const int heaviest = linear < half || items > 2 * kCus ? linear : items - 1 - (linear - half);  // index in descending weight
     const int h = heaviest % nkv, group = nq / nkv;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int col = lane & 15, g4 = lane >> 4;
-    const int r0 = (row_blocks - 1 - heaviest / nkv) * kAttnRows;
-    const int last_row = min(r0 + kAttnRows, rows) - 1;
-    const int last_key = position + last_row;  // the block's last key: every load stays at or below it
+    const int r0 = (row_blocks - 1 - heaviest / nkv) * kRows;
+    const int last_key = position + min(r0 + kRows, rows) - 1;  // the block's last key: every load stays at or below it
     const int tiles = last_key / kTile + 1;
-    const int full_tiles = (position + r0 + 1) / kTile;  // tiles every row of the block sees whole
-    const int qrow = r0 + 16 * wave + col;     // this lane's query row (B operand, output column)
+    const int wave_row = r0 + 16 * (wave / kHeadWaves), head0 = (wave % kHeadWaves) * HEADS;
+    const int full_tiles = (position + wave_row + 1) / kTile;             // tiles every row of the wave sees whole
+    const int wave_tiles = min(tiles, (position + wave_row + 15) / kTile + 1);  // tiles any of them sees
+    const int qrow = wave_row + col;  // this lane's query row (B operand, output column)
     const int qpos = position + qrow;
 
     // B operands of the scores: query row qrow of each head, dims 32 k + 8 g4 .. + 7.
-    u32x4 qb[kMaxGroup][KS];
+    u32x4 qb[HEADS][KS];
 #pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g)
+    for (int g = 0; g < HEADS; ++g)
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
-            const bool live = g < group && qrow < rows;
-            const size_t at = (static_cast<size_t>(live ? qrow : 0) * nq + h * group + (live ? g : 0)) * DH + 32 * k + 8 * g4;
+            const bool live = head0 + g < group && qrow < rows;
+            const size_t at = (static_cast<size_t>(live ? qrow : 0) * nq + h * group + (live ? head0 + g : 0)) * DH + 32 * k + 8 * g4;
             qb[g][k] = live ? *reinterpret_cast<const u32x4*>(q_rot + at) : u32x4{0u, 0u, 0u, 0u};
         }
-    // This thread's vectors of tile kt's rows (K or V cache), keys clamped to the last key.
-    auto load_rows = [&](const uint16_t* cache, int kt, u32x4 (&r)[kLoads]) {
+    // Step t < tiles is pass 1 on tile t, the others pass 2; this wave's part of a step's rows.
+    auto issue = [&](int t) {
+        const bool second = t >= tiles;
+        const int kt = second ? t - tiles : t;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
-            const int index = threadIdx.x + i * kAttnThreads, t = index / kVectors, v = index - t * kVectors;
-            const int key = min(kt * kTile + t, last_key);
-            r[i] = *reinterpret_cast<const u32x4*>(cache + (static_cast<size_t>(key) * nkv + h) * DH + 8 * v);
+            const int row0 = (wave * kLoads + i) * kRowsPerLoad, row = row0 + lane / kVectors;
+            const int chunk = (lane % kVectors) ^ (row & 7);
+            const size_t from = (static_cast<size_t>(min(kt * kTile + row, last_key)) * nkv + h) * DH + 8 * chunk;
+            load_to_lds(key_cache + from, &lds[t & 1][0][row0 * DH]);
+            if (second)
+                load_to_lds(value_cache + from, &lds[t & 1][1][row0 * DH]);
         }
     };
-    auto stage_k = [&](const u32x4 (&r)[kLoads]) {
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int index = threadIdx.x + i * kAttnThreads, t = index / kVectors, v = index - t * kVectors;
-            *reinterpret_cast<u32x4*>(ks + t * kKStride + 8 * v) = r[i];
-        }
+    // The step's tile is in LDS for every wave and the other buffer free: its next tile may load.
+    auto begin_step = [&](int t) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (t + 1 < 2 * tiles)
+            issue(t + 1);
     };
-    auto stage_v = [&](const u32x4 (&r)[kLoads]) {
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int index = threadIdx.x + i * kAttnThreads, t = index / kVectors, v = index - t * kVectors;
-            *reinterpret_cast<u32x4*>(vs + t * kVStride + 8 * v) = r[i];
-        }
+    // Two values rounded by one v_cvt_pk_bf16_f32: the empty statement keeps the pair whole, which the
+    // compiler splits where each half is used by itself, into two conversions and a shift each.
+    auto round_pair = [](float lo, float hi) {
+        uint32_t pair = pair_bf16(lo, hi);
+        asm("" : "+v"(pair));
+        return pair;
     };
-    // B operand of P V for dims 16 n .. + 15 over keys 4 g4 .. + 3 and 16 + 4 g4 .. + 3 of the
-    // 32-key step: two transposing reads (ds_read_b64_tr_b16) of the V rows as stored.  Within a
-    // 16-lane group lane j names key row 4 e + .. (e = j / 4) and dims 16 n + 4 (j % 4) .. + 3;
-    // lane `col` receives dim 16 n + col of the four rows.
-    auto v_operand = [&](int step, int n) {
-        u32x4 out;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            typedef short v4s __attribute__((ext_vector_type(4)));
-            const int row = 32 * step + 16 * h + 4 * g4 + (col >> 2);
-            const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) v4s*)(vs + row * kVStride + 16 * n + 4 * (col & 3)));
-            const uint2 pair = __builtin_bit_cast(uint2, v);
-            out[2 * h] = pair.x;
-            out[2 * h + 1] = pair.y;
-        }
-        return out;
+    // Scores of keys 32 step .. + 31 of the staged tile kt for head g: s[4 j + i] at key
+    // 64 kt + 32 step + 16 j + 4 g4 + i.
+    auto key_operand = [&](const uint16_t* ks, int subtile, int k) {
+        return *reinterpret_cast<const u32x4*>(ks + (16 * subtile + col) * DH + ((4 * k + g4) ^ (col & 7)) * 8);
     };
-    // Scores of subtile j of the staged tile kt for every head: s[g][i] at key 64 kt + 16 j + 4 g4 + i.
-    auto scores = [&](auto masked, int kt, int j, float (&s)[kMaxGroup][4]) {
-        u32x4 ka[KS];
+    auto scores = [&](auto masked, int kt, int step, const u32x4 (&ka)[2][KS], int g, float (&s)[8]) {
 #pragma unroll
-        for (int k = 0; k < KS; ++k)
-            ka[k] = *reinterpret_cast<const u32x4*>(ks + (16 * j + col) * kKStride + 32 * k + 8 * g4);
-#pragma unroll
-        for (int g = 0; g < kMaxGroup; ++g) {
+        for (int j = 0; j < 2; ++j) {
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int k = 0; k < KS; ++k)
-                acc = mfma_16x16x32_bf16(ka[k], qb[g][k], acc);
+                acc = mfma_16x16x32_bf16(ka[j][k], qb[g][k], acc);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // With head_dim 64 the scale is 2^-3: the product of a bf16 value and it is a bf16
-                // value already (short of the subnormal range), so the second rounding is the identity.
-                const float score = DH == 64 ? Bf::round(acc[i]) * 0.125f : Bf::round(Bf::round(acc[i]) * scale);
-                if constexpr (decltype(masked)::value)
-                    s[g][i] = kt * kTile + 16 * j + 4 * g4 + i <= qpos ? score : -INFINITY;
-                else
-                    s[g][i] = score;
+            for (int i = 0; i < 4; i += 2) {
+                // Rounded in pairs.  With head_dim 64 the scale is 2^-3: the product of a bf16 value
+                // and it is a bf16 value already (short of the subnormal range), so the second
+                // rounding is the identity and the product is left to the exponent's factor.
+                uint32_t pair = round_pair(acc[i], acc[i + 1]);
+                if constexpr (DH != 64)
+                    pair = round_pair(__uint_as_float(pair << 16) * scale, __uint_as_float(pair & 0xffff0000u) * scale);
+                s[4 * j + i] = __uint_as_float(pair << 16);
+                s[4 * j + i + 1] = __uint_as_float(pair & 0xffff0000u);
             }
+            if constexpr (decltype(masked)::value)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    s[4 * j + i] = kt * kTile + 32 * step + 16 * j + 4 * g4 + i <= qpos ? s[4 * j + i] : -INFINITY;
         }
     };
+    const float factor = DH == 64 ? 0.125f * kLog2e : kLog2e;  // exact: a power of two times log2 e
 
-    // Pass 1: this lane's running maximum and exp-sum per head, over its keys.
-    float m[kMaxGroup], total[kMaxGroup];
+    // Pass 1, over this lane's keys: the largest score so far, it times the factor, and the sum of
+    // 2^(s factor - reference).  A lane that has seen no key has -inf, -inf and 0.
+    float m[HEADS], reference[HEADS], total[HEADS];
 #pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g) {
-        m[g] = -INFINITY;
+    for (int g = 0; g < HEADS; ++g) {
+        m[g] = reference[g] = -INFINITY;
         total[g] = 0.0f;
     }
-    u32x4 kr[kLoads], vr[kLoads];
-    auto pass1_tile = [&](auto masked, int kt) {
-        __syncthreads();  // the previous tile's K reads are done
-        stage_k(kr);
-        load_rows(key_cache, kt + 1, kr);  // the next tile (clamped past the last) in flight
-        __syncthreads();
+    auto pass1_tile = [&](auto masked, int kt, const uint16_t* ks) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float s[kMaxGroup][4];
-            scores(masked, kt, j, s);
+        for (int step = 0; step < 2; ++step) {
+            u32x4 ka[2][KS];
 #pragma unroll
-            for (int g = 0; g < kMaxGroup; ++g) {
-                const float grown = fmaxf(m[g], fmaxf(fmaxf(s[g][0], s[g][1]), fmaxf(s[g][2], s[g][3])));
-                if constexpr (decltype(masked)::value)
-                    if (grown == -INFINITY)
-                        continue;  // every key so far masked
-                // total exp(m - grown) + e_0 + ... + e_3, the first two terms as one FMA; the factor
-                // (0 for the first subtile's m = -inf) is exactly 1 where the maximum held, and is
-                // skipped when it held in every lane of the wave.
-                const float first = exp_nonpositive(s[g][0] - grown);
-                float sum;
-                if (__builtin_amdgcn_ballot_w64(grown != m[g]) != 0)
-                    sum = fmaf(total[g], exp_nonpositive(m[g] - grown), first);
-                else
-                    sum = total[g] + first;
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int i = 1; i < 4; ++i)
-                    sum += exp_nonpositive(s[g][i] - grown);
-                total[g] = sum;
-                m[g] = grown;
+                for (int k = 0; k < KS; ++k)
+                    ka[j][k] = key_operand(ks, 2 * step + j, k);
+#pragma unroll
+            for (int g = 0; g < HEADS; ++g) {
+                float s[8];
+                scores(masked, kt, step, ka, g, s);
+                float grown = m[g];
+#pragma unroll
+                for (int i = 0; i < 8; i += 2)
+                    grown = fmaxf(grown, fmaxf(s[i], s[i + 1]));
+                // Rescaled where any lane's maximum grew (by 2^0 = 1 in the others).
+                if (__builtin_amdgcn_ballot_w64(grown > m[g]) != 0) {
+                    const float to = grown * factor;
+                    total[g] = grown > m[g] ? total[g] * __builtin_amdgcn_exp2f(reference[g] - to) : total[g];
+                    reference[g] = to;
+                    m[g] = grown;
+                }
+                float sum = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float e = __builtin_amdgcn_exp2f(fmaf(s[i], factor, -reference[g]));
+                    sum += decltype(masked)::value ? (s[i] == -INFINITY ? 0.0f : e) : e;
+                }
+                total[g] += sum;
             }
         }
     };
-    load_rows(key_cache, 0, kr);
-    int kt = 0;
-    for (; kt < full_tiles; ++kt)
-        pass1_tile(std::false_type{}, kt);
-    for (; kt < tiles; ++kt)
-        pass1_tile(std::true_type{}, kt);
-    // The four lanes of a query (lane groups g4 = 0..3) merge: M exact, S rescaled to it.
+    issue(0);
+    for (int kt = 0; kt < tiles; ++kt) {
+        begin_step(kt);
+        if (kt < full_tiles)
+            pass1_tile(std::false_type{}, kt, lds[kt & 1][0]);
+        else if (kt < wave_tiles)
+            pass1_tile(std::true_type{}, kt, lds[kt & 1][0]);
+    }
+    // The four lanes of a query (lane groups g4 = 0..3) merge, and P = 2^(s factor - shift).
+    float shift[HEADS];
 #pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g)
+    for (int g = 0; g < HEADS; ++g) {
 #pragma unroll
         for (int offset = 16; offset < 64; offset <<= 1) {
-            const float om = __shfl_xor(m[g], offset), ot = __shfl_xor(total[g], offset);
-            const float grown = fmaxf(m[g], om);
-            if (grown != -INFINITY) {
-                total[g] = total[g] * exp_nonpositive(m[g] - grown) + ot * exp_nonpositive(om - grown);
-                m[g] = grown;
+            const float other = __shfl_xor(reference[g], offset), sum = __shfl_xor(total[g], offset);
+            const float to = fmaxf(reference[g], other);
+            if (to != -INFINITY) {
+                total[g] = total[g] * __builtin_amdgcn_exp2f(reference[g] - to) + sum * __builtin_amdgcn_exp2f(other - to);
+                reference[g] = to;
             }
         }
-    float inverse[kMaxGroup];  // 1 / S, correctly rounded
-#pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g)
-        inverse[g] = 1.0f / total[g];
+        shift[g] = reference[g] + __builtin_amdgcn_logf(total[g]);
+    }
 
-    // Pass 2: P = bf16(exp(s - M) / S) as A operands, P V against the staged V rows.
-    f32x4 o[kMaxGroup][NT];
+    // Pass 2: o[g][n] += V^T P^T for dims 16 n .. + 15.
+    f32x4 o[HEADS][NT];
 #pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g)
+    for (int g = 0; g < HEADS; ++g)
 #pragma unroll
         for (int n = 0; n < NT; ++n)
             o[g][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    auto pass2_tile = [&](auto masked, int kt) {
-        __syncthreads();  // the previous tile's K and V reads are done
-        stage_k(kr);
-        stage_v(vr);
-        load_rows(key_cache, kt + 1, kr);
-        load_rows(value_cache, kt + 1, vr);
-        __syncthreads();
+    // A operand of P V for dims 16 n .. + 15 over keys 4 g4 .. + 3 and 16 + 4 g4 .. + 3 of the 32-key
+    // step: two transposing reads (ds_read_b64_tr_b16) of the V rows as stored.  Within a 16-lane
+    // group lane j names key row 4 e + .. (e = j / 4) and dims 16 n + 4 (j % 4) .. + 3; lane `col`
+    // receives dim 16 n + col of the four rows.
+    auto v_operand = [&](const uint16_t* vs, int step, int n) {
+        u32x4 r;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            typedef short v4s __attribute__((ext_vector_type(4)));
+            const int row = 32 * step + 16 * j + 4 * g4 + (col >> 2);
+            const int chunk = (2 * n + ((col & 3) >> 1)) ^ (row & 7);
+            const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) v4s*)(vs + row * DH + 8 * chunk + 4 * (col & 1)));
+            const uint2 pair = __builtin_bit_cast(uint2, v);
+            r[2 * j] = pair.x;
+            r[2 * j + 1] = pair.y;
+        }
+        return r;
+    };
+    auto pass2_tile = [&](auto masked, int kt, const uint16_t* ks, const uint16_t* vs) {
 #pragma unroll
         for (int step = 0; step < 2; ++step) {  // keys 32 step .. + 31 of the tile
-            float s0[kMaxGroup][4], s1[kMaxGroup][4];
-            scores(masked, kt, 2 * step, s0);
-            scores(masked, kt, 2 * step + 1, s1);
-            u32x4 vb[NT];
+            u32x4 ka[2][KS], va[NT];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int k = 0; k < KS; ++k)
+                    ka[j][k] = key_operand(ks, 2 * step + j, k);
 #pragma unroll
             for (int n = 0; n < NT; ++n)
-                vb[n] = v_operand(step, n);
+                va[n] = v_operand(vs, step, n);
 #pragma unroll
-            for (int g = 0; g < kMaxGroup; ++g) {
-                if (g >= group)
-                    continue;
-                float p[8];  // exp(s - M), masked keys exp(-inf) = 0; then P
+            for (int g = 0; g < HEADS; ++g) {
+                float s[8];
+                scores(masked, kt, step, ka, g, s);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    p[i] = exp_nonpositive(s0[g][i] - m[g]);
-                    p[4 + i] = exp_nonpositive(s1[g][i] - m[g]);
-                }
-                const float least = fminf(fminf(fminf(p[0], p[1]), fminf(p[2], p[3])), fminf(fminf(p[4], p[5]), fminf(p[6], p[7])));
-                if (__builtin_expect(least >= kQuotientFloor, 1)) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        p[i] = divide_by(p[i], total[g], inverse[g]);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        p[i] = p[i] / total[g];
-                }
-                // Rounded to bf16 in pairs (v_cvt_pk_bf16_f32).
-                auto pair = [](float lo, float hi) { return __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(lo), static_cast<__bf16>(hi)}); };
-                const u32x4 pa = {pair(p[0], p[1]), pair(p[2], p[3]), pair(p[4], p[5]), pair(p[6], p[7])};
+                for (int i = 0; i < 8; ++i)
+                    s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], factor, -shift[g]));
+                const u32x4 p = pack_bf16(s);
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
-                    o[g][n] = mfma_16x16x32_bf16(pa, vb[n], o[g][n]);
+                    o[g][n] = mfma_16x16x32_bf16(va[n], p, o[g][n]);
             }
         }
     };
-    load_rows(key_cache, 0, kr);
-    load_rows(value_cache, 0, vr);
-    for (kt = 0; kt < full_tiles; ++kt)
-        pass2_tile(std::false_type{}, kt);
-    for (; kt < tiles; ++kt)
-        pass2_tile(std::true_type{}, kt);
-    // o[g][n]: lane l holds query rows r0 + 16 wave + 4 g4 + i, dim 16 n + col.
+    for (int kt = 0; kt < tiles; ++kt) {
+        const int t = tiles + kt;
+        begin_step(t);
+        if (kt < full_tiles)
+            pass2_tile(std::false_type{}, kt, lds[t & 1][0], lds[t & 1][1]);
+        else if (kt < wave_tiles)
+            pass2_tile(std::true_type{}, kt, lds[t & 1][0], lds[t & 1][1]);
+    }
+    // o[g][n]: lane l holds query row qrow, dims 16 n + 4 g4 .. + 3.
+    if (qrow < rows)
 #pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = r0 + 16 * wave + 4 * g4 + i;
-            if (g < group && r < rows)
+        for (int g = 0; g < HEADS; ++g)
+            if (head0 + g < group)
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
-                    out[(static_cast<size_t>(r) * nq + h * group + g) * DH + 16 * n + col] = bits16(Bf::round(o[g][n][i]));
-        }
+                    *reinterpret_cast<uint2*>(out + (static_cast<size_t>(qrow) * nq + h * group + head0 + g) * DH + 16 * n + 4 * g4) =
+                        uint2{pair_bf16(o[g][n][0], o[g][n][1]), pair_bf16(o[g][n][2], o[g][n][3])};
 }
 
 // The tile shapes of the GEMM, and the time in us a 64-wide K step of one takes a CU that runs one
@@ -477,7 +480,6 @@ struct TileShape {
 constexpr TileShape kTileShapes[] = {{256, 256, 2.03f, 0.0f}, {128, 128, 0.85f, 1.1f}, {128, 64, 0.52f, 0.74f}, {64, 64, 0.29f, 0.46f}};
 constexpr float kBlockStart = 2.4f;         // us a block takes besides its K steps
 constexpr float kPartialRate = 3.1e6f;      // bytes per us that partial sums are written and read back at
-constexpr int kCus = 256;
 constexpr size_t kPartialFloats = 16u << 20;  // 64 MiB of partial sums
 
 struct Tiling {
@@ -594,6 +596,28 @@ Views views(void* buffer, const ti_model_shape& s, size_t rows)
     return v;
 }
 
+// Attention of `rows` query rows: the most heads a wave (K and V operands read once for all of them)
+// that leave two blocks a CU; fewer, and more blocks of fewer rows, for shorter prompts.
+template <int DH, int HEADS = kMaxGroup>
+void attend_heads(hipStream_t stream, const uint16_t* q, int position, int rows, int nq, int nkv, const uint16_t* k, const uint16_t* v,
+                  float scale, uint16_t* out)
+{
+    const int blocks = (rows + 16 * HEADS - 1) / (16 * HEADS);
+    if constexpr (HEADS > 1)
+        if (blocks * nkv < 2 * kCus)
+            return attend_heads<DH, HEADS / 2>(stream, q, position, rows, nq, nkv, k, v, scale, out);
+    hipLaunchKernelGGL((attention_tiles<DH, HEADS>), dim3(blocks, nkv), dim3(kAttnThreads), 0, stream, q, position, rows, nq, nkv, k,
+                       v, scale, out);
+}
+void attend(hipStream_t stream, const uint16_t* q, int position, int rows, int nq, int nkv, int dh, const uint16_t* k,
+            const uint16_t* v, float scale, uint16_t* out)
+{
+    if (dh == 64)
+        attend_heads<64>(stream, q, position, rows, nq, nkv, k, v, scale, out);
+    else
+        attend_heads<128>(stream, q, position, rows, nq, nkv, k, v, scale, out);
+}
+
 // Enqueues X W^T of x [m][k] and w [n][k] into rows of c, or as partial sums; returns where the
 // product is.  With a residual (row stride n), c receives bf16(bf16(sum) + residual) unless the
 // sums are partial: the kernel that adds those adds the residual too.
@@ -674,13 +698,7 @@ int MatrixPrefill::layer(hipStream_t stream, void* kv, int layer, int position, 
         rope(std::integral_constant<int, 128>{});
     if (!last) {
         const float scale = 1.0f / sqrtf(static_cast<float>(dh));
-        const dim3 attention_grid((rows + kAttnRows - 1) / kAttnRows, nkv);
-        if (dh == 64)
-            hipLaunchKernelGGL(attention_tiles<64>, attention_grid, dim3(kAttnThreads), 0, stream, v.q, position, rows, nq, nkv,
-                               cache + w.key, cache + w.value, scale, v.attention);
-        else
-            hipLaunchKernelGGL(attention_tiles<128>, attention_grid, dim3(kAttnThreads), 0, stream, v.q, position, rows, nq, nkv,
-                               cache + w.key, cache + w.value, scale, v.attention);
+        attend(stream, v.q, position, rows, nq, nkv, dh, cache + w.key, cache + w.value, scale, v.attention);
         const GemmRows projected = gemm(stream, v.attention, rows, qw, base + w.Wo, d, v.x, v.r, d, v.partial);
         norm(projected, v.x, v.r, base + w.ffn_norm);
         GemmArgs ffn{v.u, base + w.Wgate, base + w.Wup, nullptr, v.product, nullptr, rows, f, d, f, 1, 0, 0};
