@@ -45,7 +45,10 @@ def check(tmp_path, hidden, intermediate, heads, kv_heads, length, std):
 
 
 @pytest.mark.parametrize("hidden,intermediate,heads,kv_heads,length,std", [
-    (256, 544, 4, 1, 66, 0.08),       # 65 rows; down projection over 544 = 17 x 32
+    (256, 512, 4, 1, 4, 0.08),        # the shortest prompt that is prefilled with matrices: 3 rows
+    (2048, 8192, 32, 8, 17, 0.02),    # 16 rows
+    (256, 544, 4, 1, 65, 0.08),       # 64 rows; down projection over 544 = 17 x 32
+    (256, 544, 4, 1, 66, 0.08),       # 65 rows
     (128, 32, 2, 1, 129, 0.12),       # 128 rows; gate/up and down narrower than any tile
     (256, 512, 4, 2, 130, 0.08),      # 129 rows
     (512, 1056, 8, 2, 257, 0.05),     # 256 rows; 33 x 32

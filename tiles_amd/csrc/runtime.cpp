@@ -202,7 +202,7 @@ struct Context {
     DeviceBuffer head_hidden, head_token;  // LM-head step: input vector and selected token
     DeviceBuffer timeline;
     bool timeline_enabled = false;
-    // Prompts longer than one worker launch prefill all but their last token with matrices
+    // Prompts of MatrixPrefill::kMinPrompt tokens or more prefill all but their last with matrices
     // (bf16 decoder stacks; the rest go through the worker one position per step).
     bool matrix_prefill = true;
     std::unique_ptr<MatrixPrefill> matrix;
@@ -474,7 +474,7 @@ struct Context {
         try {
             stage_input(ids, count);
             const int n = static_cast<int>(count);
-            if (matrix_prefill && n > TI_MAX_LAUNCH_STEPS && MatrixPrefill::supports(model->view)) {
+            if (matrix_prefill && n >= MatrixPrefill::kMinPrompt && MatrixPrefill::supports(model->view)) {
                 // The worker decodes the last token: its step leaves the greedy candidates and
                 // diagnostics a generation or collect() continues from.
                 if (!matrix)

@@ -365,7 +365,7 @@ class SequenceContext:
         return Ticket(self, handle, "lm_head", 1)
 
     def set_matrix_prefill(self, enabled: bool) -> None:
-        """Prefills of more than 64 tokens on bf16 stacks run all but the last token as matrices
+        """Prefills of 4 tokens or more on bf16 stacks run all but the last token as matrices
         (on by default); off, every token goes through the worker."""
         _check(library().ti_context_set_matrix_prefill(self._handle, int(enabled)))
 
