@@ -45,7 +45,7 @@ def check(tmp_path, hidden, intermediate, heads, kv_heads, length, std):
 
 
 @pytest.mark.parametrize("hidden,intermediate,heads,kv_heads,length,std", [
-    (256, 512, 4, 1, 4, 0.08),        # the shortest prompt that is prefilled with matrices: 3 rows
+    (256, 512, 4, 1, 3, 0.08),        # the shortest prompt that is prefilled with matrices
     (2048, 8192, 32, 8, 17, 0.02),    # 16 rows
     (256, 544, 4, 1, 65, 0.08),       # 64 rows; down projection over 544 = 17 x 32
     (256, 544, 4, 1, 66, 0.08),       # 65 rows
@@ -69,3 +69,32 @@ def test_matrix_prefill_attention_forms(tmp_path, hidden, intermediate, heads, k
     """The attention's heads per wave (as many as leave two blocks a CU), query groups smaller than a
     wave takes, and both head widths."""
     check(tmp_path, hidden, intermediate, heads, kv_heads, length, std)
+
+
+def test_prompt_in_many_parts_then_generation(tmp_path):
+    """60 prompts of 4 to 7 tokens queued on one context (each ends with a launch of the logits tasks
+    alone, which takes one step's exchange epochs), then 70 generated tokens (two launches), beside a
+    context whose every token goes through the worker.  The logits of both after the same 330 + 70
+    tokens are within 2^-6 of their RMS: 2 layers' roundings (2^-7, above) on either side."""
+    dims = dict(hidden_size=256, intermediate_size=512, num_attention_heads=4, num_key_value_heads=1, head_dim=64, max_context=420)
+    spec = P.StackSpec(P.BlockSpec(**dims), 2, 512, True)
+    K.build_stack_package(spec, K.random_weights(spec, seed=5, std=0.08), probe.probe_library(), tmp_path / "pkg", "bfloat16")
+    model = R.DecoderModel(R.load_plan(tmp_path / "pkg"))
+    parts = [np.random.default_rng(i).integers(0, 512, 4 + i % 4).tolist() for i in range(60)]
+    matrix, worker = model.create_context(), model.create_context()
+    worker.set_matrix_prefill(False)
+    tickets = [matrix.enqueue_prefill(p, logits=True) for p in parts]
+    last = matrix.collect(tickets[-1])["logits"]
+    generated = matrix.wait(matrix.enqueue_generate(70)).generated
+    after = matrix.collect(matrix.enqueue_decode(generated[0], logits=True))["logits"]
+    for p in parts[:-1]:
+        worker.enqueue_prefill(p)
+    want = worker.collect(worker.enqueue_prefill(parts[-1], logits=True))["logits"]
+    assert np.argmax(last) == generated[0] and len(generated) == 70
+    for first in range(0, 70, 64):  # the same tokens, forced
+        worker.enqueue_prefill(generated[first:first + 64])
+    want_after = worker.collect(worker.enqueue_decode(generated[0], logits=True))["logits"]
+    for got, expected in ((last, want), (after, want_after)):
+        off = float(np.sqrt(((got - expected) ** 2).mean() / (expected ** 2).mean()))
+        print(f"off by {off:.5f} of the RMS", flush=True)
+        assert off <= 2.0 ** -6

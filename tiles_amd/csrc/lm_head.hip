@@ -1,6 +1,6 @@
 // The LM-head step alone: a given hidden vector through the final RMSNorm, the LM-head GEMV and
-// greedy selection, run by the decode worker's own logits tasks (op_logits), so that the step is
-// timed as one launch of the kernel that runs it inside every decode step.  The worker launch
+// greedy selection, run by the decode worker's own logits tasks (op_logits): the end of a matrix
+// prefill, and, timed as one launch of the kernel that runs it inside every decode step, a benchmark.  The worker launch
 // takes a program of only the package's logits tasks; its input comes from the exchange, where
 // a seed kernel publishes the vector as the last layer's output of the launch's first step.
 
@@ -59,11 +59,11 @@ __global__ void __launch_bounds__(kSelectThreads) select_candidate(const ti_cand
 
 } // namespace
 
-int enqueue_lm_head_step(hipStream_t stream, const ti_worker_program_view& head, const ti_worker_buffers& b, const void* hidden,
-                         ti_token_id* token, hipEvent_t worker_start, hipEvent_t worker_end)
+int enqueue_logits(hipStream_t stream, const ti_worker_program_view& head, const ti_worker_buffers& b, const void* hidden,
+                   hipEvent_t worker_start, hipEvent_t worker_end)
 {
-    if (!hidden || !token || !b.exchange || !b.selection || head.selection_slots < 1)
-        return fail(TI_ERR_INVALID_ARGUMENT, "LM-head step needs a hidden vector, a token slot, the exchange and candidates");
+    if (!hidden || !b.exchange || !b.selection || head.selection_slots < 1)
+        return fail(TI_ERR_INVALID_ARGUMENT, "LM-head step needs a hidden vector, the exchange and candidates");
     const int d = head.shape.hidden_size;
     const int layers = head.stack.layers;
     if (d < 1 || layers < 1)
@@ -88,8 +88,19 @@ int enqueue_lm_head_step(hipStream_t stream, const ti_worker_program_view& head,
         return code;
     if (worker_end && (e = hipEventRecord(worker_end, stream)) != hipSuccess)
         return hip_fail(e, "LM-head timing event");
+    return TI_OK;
+}
+
+int enqueue_lm_head_step(hipStream_t stream, const ti_worker_program_view& head, const ti_worker_buffers& b, const void* hidden,
+                         ti_token_id* token, hipEvent_t worker_start, hipEvent_t worker_end)
+{
+    if (!token)
+        return fail(TI_ERR_INVALID_ARGUMENT, "LM-head step needs a token slot");
+    const int code = enqueue_logits(stream, head, b, hidden, worker_start, worker_end);
+    if (code != TI_OK)
+        return code;
     hipLaunchKernelGGL(select_candidate, dim3(1), dim3(kSelectThreads), 0, stream, b.selection, head.selection_slots, token);
-    e = hipGetLastError();
+    const hipError_t e = hipGetLastError();
     return e == hipSuccess ? TI_OK : hip_fail(e, "LM-head selection launch");
 }
 

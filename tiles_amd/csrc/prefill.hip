@@ -646,32 +646,71 @@ GemmRows gemm(hipStream_t stream, const uint16_t* x, int m, int k, const uint16_
 }
 } // namespace
 
+namespace {
+// out = RMSNorm(x), x first completed (into x, from `residual`) when the GEMM left parts.
+void norm(hipStream_t stream, const GemmRows& sums, const uint16_t* residual, uint16_t* x, const uint16_t* scale, int rows, int d,
+          float eps, uint16_t* out)
+{
+    with_splits(sums.splits, [&](auto n) {
+        hipLaunchKernelGGL(norm_rows<n>, dim3(rows), dim3(kRowThreads), 0, stream, sums, n > 1 ? residual : x, scale, d, eps, x, out);
+    });
+}
+void rope(hipStream_t stream, const GemmRows& qkv, int rows, int position, const float* frequencies, int nq, int nkv, int dh,
+          uint16_t* q_rot, uint16_t* key_cache, uint16_t* value_cache)
+{
+    auto launch = [&](auto head_dim) {
+        with_splits(qkv.splits, [&](auto n) {
+            hipLaunchKernelGGL((rope_rows<head_dim, n>), dim3(rows), dim3(kRowThreads), 0, stream, qkv, position, frequencies, nq,
+                               nkv, q_rot, key_cache, value_cache);
+        });
+    };
+    if (dh == 64)
+        launch(std::integral_constant<int, 64>{});
+    else
+        launch(std::integral_constant<int, 128>{});
+}
+} // namespace
+
+const uint16_t* MatrixPrefill::weights(int layer) const
+{
+    return static_cast<const uint16_t*>(p_.weights) + p_.stack.layer_weights_offset +
+           static_cast<size_t>(layer) * p_.stack.layer_weight_stride;
+}
+
+// From the attention output of `rows` rows (their layer input in x from row `first_row`) to the layer's
+// output, in the same rows of x, and its RMSNorm with `next_norm` in u.
+void MatrixPrefill::feed_forward(hipStream_t stream, int layer, int rows, int first_row, const uint16_t* next_norm)
+{
+    const ti_model_shape& s = p_.shape;
+    const int d = s.hidden_size, f = s.intermediate_size, qw = s.query_heads * s.head_dim;
+    const ti_layer_layout& w = p_.layout;
+    const uint16_t* base = weights(layer);
+    const Views v = views(buffer_, s, kChunkRows);
+    uint16_t* x = v.x + static_cast<size_t>(first_row) * d;
+    const float eps = p_.numeric.rms_norm_eps;
+    const GemmRows projected = gemm(stream, v.attention, rows, qw, base + w.Wo, d, x, v.r, d, v.partial);
+    norm(stream, projected, x, v.r, base + w.ffn_norm, rows, d, eps, v.u);
+    GemmArgs ffn{v.u, base + w.Wgate, base + w.Wup, nullptr, v.product, nullptr, rows, f, d, f, 1, 0, 0};
+    launch_shape<GemmOut::kSilu>(stream, choose_tiling(rows, 2 * f, d, false).shape, ffn);
+    // Wdown row-major [hidden][intermediate] on the device (ti_relayout_weights).
+    const GemmRows down = gemm(stream, v.product, rows, f, base + w.Wdown, d, v.r, x, d, v.partial);
+    norm(stream, down, v.r, x, next_norm, rows, d, eps, v.u);
+}
+
 int MatrixPrefill::layer(hipStream_t stream, void* kv, int layer, int position, int rows)
 {
     const ti_model_shape& s = p_.shape;
-    const int d = s.hidden_size, f = s.intermediate_size, dh = s.head_dim, nq = s.query_heads, nkv = s.kv_heads;
+    const int d = s.hidden_size, dh = s.head_dim, nq = s.query_heads, nkv = s.kv_heads;
     const int qw = nq * dh, kvw = nkv * dh;
     const Views v = views(buffer_, s, kChunkRows);
     const ti_layer_layout& w = p_.layout;
-    auto weights = [&](int of) {
-        return static_cast<const uint16_t*>(p_.weights) + p_.stack.layer_weights_offset +
-               static_cast<size_t>(of) * p_.stack.layer_weight_stride;
-    };
     const uint16_t* base = weights(layer);
     uint16_t* cache = static_cast<uint16_t*>(kv) + static_cast<size_t>(layer) * p_.stack.layer_kv_stride;
-    const float eps = p_.numeric.rms_norm_eps;
-    // out = RMSNorm(x), x first completed (into sum_out) by the residual when the GEMM left parts.
-    auto norm = [&](const GemmRows& sums, const uint16_t* residual, uint16_t* sum_out, const uint16_t* scale) {
-        with_splits(sums.splits, [&](auto n) {
-            hipLaunchKernelGGL(norm_rows<n>, dim3(rows), dim3(kRowThreads), 0, stream, sums, n > 1 ? residual : sum_out, scale, d,
-                               eps, sum_out, v.u);
-        });
-    };
 
     if (layer == 0)
-        norm({v.x, nullptr, 1, 0}, nullptr, v.x, base + w.attn_norm);
-    // The prompt's last position goes through the worker, and the positions here are read again only
-    // as cache rows: the last layer ends with its K and V.
+        norm(stream, {v.x, nullptr, 1, 0}, nullptr, v.x, base + w.attn_norm, rows, d, p_.numeric.rms_norm_eps, v.u);
+    // Of the last layer's positions only the cache rows are read again (and, where last_row follows,
+    // the last one's output): it ends with its K and V.
     const bool last = layer + 1 == p_.stack.layers;
     const int first_row = last ? qw : 0, width = (last ? 0 : qw) + 2 * kvw;
     GemmRows qkv{v.qkv, nullptr, 1, 0};
@@ -685,32 +724,36 @@ int MatrixPrefill::layer(hipStream_t stream, void* kv, int layer, int position, 
         gemm(stream, v.u, rows, d, base + w.Wk, kvw, nullptr, v.qkv + width - 2 * kvw, width, nullptr);
         gemm(stream, v.u, rows, d, base + w.Wv, kvw, nullptr, v.qkv + width - kvw, width, nullptr);
     }
-    const int rotated_queries = last ? 0 : nq;
-    auto rope = [&](auto head_dim) {
-        with_splits(qkv.splits, [&](auto n) {
-            hipLaunchKernelGGL((rope_rows<head_dim, n>), dim3(rows), dim3(kRowThreads), 0, stream, qkv, position,
-                               p_.rotary_frequencies, rotated_queries, nkv, v.q, cache + w.key, cache + w.value);
-        });
-    };
-    if (dh == 64)
-        rope(std::integral_constant<int, 64>{});
-    else
-        rope(std::integral_constant<int, 128>{});
+    rope(stream, qkv, rows, position, p_.rotary_frequencies, last ? 0 : nq, nkv, dh, v.q, cache + w.key, cache + w.value);
     if (!last) {
-        const float scale = 1.0f / sqrtf(static_cast<float>(dh));
-        attend(stream, v.q, position, rows, nq, nkv, dh, cache + w.key, cache + w.value, scale, v.attention);
-        const GemmRows projected = gemm(stream, v.attention, rows, qw, base + w.Wo, d, v.x, v.r, d, v.partial);
-        norm(projected, v.x, v.r, base + w.ffn_norm);
-        GemmArgs ffn{v.u, base + w.Wgate, base + w.Wup, nullptr, v.product, nullptr, rows, f, d, f, 1, 0, 0};
-        launch_shape<GemmOut::kSilu>(stream, choose_tiling(rows, 2 * f, d, false).shape, ffn);
-        // Wdown row-major [hidden][intermediate] on the device (ti_relayout_weights).
-        const GemmRows down = gemm(stream, v.product, rows, f, base + w.Wdown, d, v.r, v.x, d, v.partial);
-        norm(down, v.r, v.x, weights(layer + 1) + w.attn_norm);
+        attend(stream, v.q, position, rows, nq, nkv, dh, cache + w.key, cache + w.value, 1.0f / sqrtf(static_cast<float>(dh)),
+               v.attention);
+        feed_forward(stream, layer, rows, 0, weights(layer + 1) + w.attn_norm);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return hip_fail(e, "prefill kernel launch");
     return TI_OK;
+}
+
+int MatrixPrefill::last_row(hipStream_t stream, void* kv, int position, const void** hidden)
+{
+    if (!buffer_ || rows_ < 1 || position < rows_ - 1)
+        return fail(TI_ERR_INVALID_ARGUMENT, "no prefilled position to finish");
+    const ti_model_shape& s = p_.shape;
+    const int d = s.hidden_size, dh = s.head_dim, nq = s.query_heads, nkv = s.kv_heads, layer = p_.stack.layers - 1;
+    const Views v = views(buffer_, s, kChunkRows);
+    const ti_layer_layout& w = p_.layout;
+    const uint16_t* cache = static_cast<const uint16_t*>(kv) + static_cast<size_t>(layer) * p_.stack.layer_kv_stride;
+    const size_t row = rows_ - 1;
+    const GemmRows q = gemm(stream, v.u + row * d, 1, d, weights(layer) + w.Wq, nq * dh, nullptr, v.qkv, nq * dh, v.partial);
+    rope(stream, q, 1, position, p_.rotary_frequencies, nq, 0, dh, v.q, nullptr, nullptr);
+    attend(stream, v.q, position, 1, nq, nkv, dh, cache + w.key, cache + w.value, 1.0f / sqrtf(static_cast<float>(dh)), v.attention);
+    const uint16_t* final_norm = static_cast<const uint16_t*>(p_.weights) + p_.stack.final_norm_offset;
+    feed_forward(stream, layer, 1, static_cast<int>(row), final_norm);  // the norm's output is not used
+    *hidden = v.x + row * d;
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TI_OK : hip_fail(e, "prefill kernel launch");
 }
 
 int MatrixPrefill::enqueue(hipStream_t stream, void* kv, const ti_token_id* tokens, int position, int count)
@@ -732,7 +775,7 @@ int MatrixPrefill::enqueue(hipStream_t stream, void* kv, const ti_token_id* toke
     const Views v = views(buffer_, p_.shape, kChunkRows);
     const uint16_t* embedding = static_cast<const uint16_t*>(p_.weights) + p_.stack.embedding_offset;
     for (int first = 0; first < count; first += kChunkRows) {
-        const int rows = std::min(kChunkRows, count - first);
+        const int rows = rows_ = std::min(kChunkRows, count - first);
         hipLaunchKernelGGL(gather_rows, dim3(rows), dim3(kRowThreads), 0, stream, embedding, tokens + first, p_.shape.hidden_size,
                            v.x);
         for (int layer = 0; layer < p_.stack.layers; ++layer) {

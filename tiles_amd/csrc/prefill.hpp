@@ -15,10 +15,15 @@ class MatrixPrefill {
   public:
     // Positions per pass through the layers: the activation buffers hold this many rows.
     static constexpr int kChunkRows = 4096;
-    // The shortest prompt that takes this path: its kernels read every weight once, about as long as two
-    // worker steps take (Llama-3.2-1B: 4 tokens 1.77 ms against 2.46 through the worker, 37 tokens 1.80
-    // against 19.2; 3 tokens 1.97 through the worker).
-    static constexpr int kMinPrompt = 4;
+    // The shortest prompt that takes this path: its kernels read every weight once, in about the time of
+    // two worker steps (Llama-3.2-1B: 3 tokens 1.34 ms against 1.97 through the worker, 37 tokens 1.45
+    // against 19.2, 2 tokens 1.39 against 1.45; two of its layers alone: 3 tokens 0.68 against 0.77).
+    static constexpr int kMinPrompt = 3;
+    // Positions up to which the prompt's last token goes through the matrices as well (last_row) and its
+    // hidden vector to the LM head, instead of a worker step, which reads every weight again: 0.4-0.5 ms
+    // less from 3 tokens (1.34 ms against 1.71) to 1,024 (3.52 against 4.00).  Its attention is one pass
+    // over the cache by a block a K/V head, which grows with the position; the worker splits it.
+    static constexpr int kLastRowPositions = 1024;
 
     explicit MatrixPrefill(const ti_worker_program_view& program);
     ~MatrixPrefill();
@@ -33,12 +38,18 @@ class MatrixPrefill {
     // positions go into `kv`.  The positions before `position` must already be in the cache.
     // Returns a TI_* code; the message is in ti_last_error_message().
     int enqueue(hipStream_t stream, void* kv, const ti_token_id* tokens, int position, int count);
+    // After enqueue: the rest of the last layer for the last of its positions.  `hidden` receives that
+    // position's output of the stack (device memory of this object, good until the next enqueue).
+    int last_row(hipStream_t stream, void* kv, int position, const void** hidden);
 
   private:
     ti_worker_program_view p_;
     void* buffer_ = nullptr;  // every activation buffer, kChunkRows rows each
     size_t buffer_bytes_ = 0;
+    int rows_ = 0;  // of the last pass: positions it left in the activation buffers
     int layer(hipStream_t stream, void* kv, int layer, int position, int rows);
+    const uint16_t* weights(int layer) const;
+    void feed_forward(hipStream_t stream, int layer, int rows, int first_row, const uint16_t* next_norm);
 };
 
 } // namespace tiles

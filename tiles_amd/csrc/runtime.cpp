@@ -210,6 +210,7 @@ struct Context {
     PinnedBuffer ring;
     size_t ring_cursor = 0;
     uint32_t epoch = 1;
+    uint32_t logits_epochs = 0;  // epochs that logits launches took since the last whole launch
     int queued_position = 0;
     std::shared_ptr<Ticket> pending;
     bool valid = true;
@@ -341,7 +342,9 @@ struct Context {
         return b;
     }
 
-    void advance_epoch()
+    void advance_epoch() { advance_epoch(ti_epochs_per_launch(model->meta.stack.layers)); }
+    // `by` at most one launch's epochs.
+    void advance_epoch(uint32_t by)
     {
         const uint32_t step = ti_epochs_per_launch(model->meta.stack.layers);
         if (epoch > 0xffffffffu - 2 * step) {
@@ -356,8 +359,29 @@ struct Context {
                   "clear exchange");
             epoch = 1;
         } else {
-            epoch += step;
+            epoch += by;
         }
+    }
+
+    // Whether a launch of the logits tasks alone may run now.  It takes one step's epochs and leaves
+    // the other exchange vectors as the last whole launch wrote them, so each such launch makes them
+    // one step older; the next whole launch writes every element in its first step, and until then a
+    // stale bf16 element's 16-bit tag must not come round to one that is awaited.
+    bool logits_launch_fits() const
+    {
+        const uint32_t step = epochs_per_step(model->meta.stack.layers);
+        return model->head_tasks > 0 && ti_epochs_per_launch(model->meta.stack.layers) + logits_epochs + 2 * step < 65535u;
+    }
+
+    // The LM head and greedy candidates for `hidden`, the stack's output at the last position.
+    void launch_logits(const void* hidden)
+    {
+        ti_worker_buffers b = worker_buffers(false);
+        b.epoch = epoch;
+        check_ti(enqueue_logits(stream, model->head_view, b, hidden, nullptr, nullptr));
+        const uint32_t step = epochs_per_step(model->meta.stack.layers);
+        advance_epoch(step);
+        logits_epochs += step;
     }
 
     // Decodes `steps` positions from `position` in launches of at most 64 steps; `epochs`, when
@@ -380,6 +404,7 @@ struct Context {
             ti_token_input token{-1, ids ? ids + first : nullptr, count};
             check_ti(ti_enqueue_worker(stream, &model->view, &b, position + first, token, selection));
             advance_epoch();
+            logits_epochs = 0;
         }
     }
 
@@ -475,12 +500,21 @@ struct Context {
             stage_input(ids, count);
             const int n = static_cast<int>(count);
             if (matrix_prefill && n >= MatrixPrefill::kMinPrompt && MatrixPrefill::supports(model->view)) {
-                // The worker decodes the last token: its step leaves the greedy candidates and
-                // diagnostics a generation or collect() continues from.
                 if (!matrix)
                     matrix = std::make_unique<MatrixPrefill>(model->view);
-                check_ti(matrix->enqueue(stream, kv.ptr, tokens.as<ti_token_id>(), start, n - 1));
-                launch(start + n - 1, tokens.as<ti_token_id>() + n - 1, 1, diag.block_outputs != 0, ti_selection{});
+                // The last token leaves the logits and greedy candidates that a generation or collect()
+                // continues from: through the matrices and the logits tasks, or, where its position
+                // is far, or the diagnostics or the timeline of a whole step are asked for, through a
+                // worker step.
+                if (start + n <= MatrixPrefill::kLastRowPositions && !diag.block_outputs && !timeline_enabled && logits_launch_fits()) {
+                    const void* hidden = nullptr;
+                    check_ti(matrix->enqueue(stream, kv.ptr, tokens.as<ti_token_id>(), start, n));
+                    check_ti(matrix->last_row(stream, kv.ptr, start + n - 1, &hidden));
+                    launch_logits(hidden);
+                } else {
+                    check_ti(matrix->enqueue(stream, kv.ptr, tokens.as<ti_token_id>(), start, n - 1));
+                    launch(start + n - 1, tokens.as<ti_token_id>() + n - 1, 1, diag.block_outputs != 0, ti_selection{});
+                }
             } else {
                 launch(start, tokens.as<ti_token_id>(), n, diag.block_outputs != 0, ti_selection{});
             }
@@ -579,6 +613,7 @@ struct Context {
             // As a reset leaves the context: no exchange word of these launches stays behind.
             check(hipMemsetAsync(exchange.ptr, 0, exchange.bytes, stream), "reset exchange");
             epoch = 1;
+            logits_epochs = 0;
         } catch (...) {
             valid = false;
             (void)hipStreamSynchronize(stream);
@@ -597,6 +632,7 @@ struct Context {
             // A failed launch may leave partial exchange state (attention merge counts).
             check(hipMemsetAsync(exchange.ptr, 0, exchange.bytes, stream), "reset exchange");
             epoch = 1;
+            logits_epochs = 0;
             finish_ticket(t, {});
             queued_position = 0;
             valid = true;

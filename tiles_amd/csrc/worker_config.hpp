@@ -206,11 +206,15 @@ int launch_worker_f32(hipStream_t stream, const ti_worker_program_view& p, const
 // launch from another stream to complete (two launches cannot share the device).
 int enqueue_worker(hipStream_t s, const ti_worker_program_view& program, const ti_worker_buffers& buffers, int32_t position,
                    ti_token_input token, ti_selection selection, bool order_streams);
-// The LM-head step alone (lm_head.hip): `hidden` (device, hidden_size elements of the weight
-// type) published as the last layer's output of a launch at buffers.epoch, one step of `head`
-// (a program of the package's logits tasks only), then greedy selection of the candidates into
-// `token` (device).  The launch uses exchange epochs [buffers.epoch, + ti_epochs_per_launch).
-// worker_start / worker_end (optional) are recorded around the worker launch alone.
+// The LM head on a given vector (lm_head.hip): `hidden` (device, hidden_size elements of the weight
+// type) published as the last layer's output of a launch at buffers.epoch, then one step of `head`
+// (a program of the package's logits tasks only), which leaves logits and candidates as a decode step
+// does.  The launch uses the exchange epochs of its one step.  worker_start / worker_end (optional)
+// are recorded around the worker launch alone.
+int enqueue_logits(hipStream_t stream, const ti_worker_program_view& head, const ti_worker_buffers& buffers, const void* hidden,
+                   hipEvent_t worker_start, hipEvent_t worker_end);
+// The isolated LM-head step: enqueue_logits, then greedy selection of the candidates into `token`
+// (device).
 int enqueue_lm_head_step(hipStream_t stream, const ti_worker_program_view& head, const ti_worker_buffers& buffers,
                          const void* hidden, ti_token_id* token, hipEvent_t worker_start, hipEvent_t worker_end);
 std::vector<const void*> worker_functions_bf16();

@@ -365,8 +365,8 @@ class SequenceContext:
         return Ticket(self, handle, "lm_head", 1)
 
     def set_matrix_prefill(self, enabled: bool) -> None:
-        """Prefills of 4 tokens or more on bf16 stacks run all but the last token as matrices
-        (on by default); off, every token goes through the worker."""
+        """Prefills of 3 tokens or more on bf16 stacks run as matrices (on by default; past position
+        1024 all but their last token); off, every token goes through the worker."""
         _check(library().ti_context_set_matrix_prefill(self._handle, int(enabled)))
 
     def set_timeline(self, enabled: bool) -> None:
