@@ -5,10 +5,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <bit>
 #include <cstdio>
 #include <cstring>
 #include <deque>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -80,6 +82,65 @@ struct PinnedBuffer {
         return *this;
     }
     template <typename T> T* as() const { return static_cast<T*>(ptr); }
+};
+
+// Small pinned buffers that a context's tickets take and give back: allocating and freeing one costs
+// 25-40 us, and a request takes up to four.  Every buffer receives device-to-host copies on the
+// context's one stream only and is read after its ticket's event, so a copy still queued for a ticket
+// that was dropped lands before the next taker's.  Shared by the context and its tickets (which may
+// outlive it, on any thread), bounded, and freed with the last of them.
+class PinnedPool {
+  public:
+    static constexpr size_t kLargest = 1u << 20, kMostBytes = 8u << 20;
+    PinnedBuffer take(size_t n)
+    {
+        if (n > kLargest)
+            return PinnedBuffer(n);
+        const size_t size = std::bit_ceil(std::max<size_t>(n, 64));
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            for (auto it = free_.begin(); it != free_.end(); ++it)
+                if (it->bytes == size) {
+                    PinnedBuffer found = std::move(*it);
+                    free_.erase(it);
+                    held_ -= size;
+                    return found;
+                }
+        }
+        return PinnedBuffer(size);
+    }
+    void give(PinnedBuffer&& buffer)
+    {
+        std::lock_guard<std::mutex> lock(mutex_);
+        if (buffer.bytes > kLargest || held_ + buffer.bytes > kMostBytes)
+            return;  // freed by the caller's destructor
+        held_ += buffer.bytes;
+        free_.push_back(std::move(buffer));
+    }
+
+  private:
+    std::mutex mutex_;
+    std::vector<PinnedBuffer> free_;
+    size_t held_ = 0;
+};
+
+// A buffer of the pool for as long as it lives.
+struct PooledBuffer {
+    PooledBuffer(std::shared_ptr<PinnedPool> from, size_t n) : pool(std::move(from)), buffer(pool->take(n)), ptr(buffer.ptr), bytes(n) {}
+    ~PooledBuffer()
+    {
+        try {
+            pool->give(std::move(buffer));
+        } catch (...) {  // out of memory for the list: the buffer is freed instead
+        }
+    }
+    PooledBuffer(const PooledBuffer&) = delete;
+    PooledBuffer& operator=(const PooledBuffer&) = delete;
+    template <typename T> T* as() const { return static_cast<T*>(ptr); }
+    std::shared_ptr<PinnedPool> pool;
+    PinnedBuffer buffer;
+    void* ptr;
+    size_t bytes;
 };
 
 } // namespace
@@ -172,9 +233,9 @@ struct Ticket {
     size_t input_begin = 0, input_count = 0;
     bool generation = false;
     int start_position = 0, requested = 0;
-    std::unique_ptr<PinnedBuffer> output, status, control;
+    std::unique_ptr<PooledBuffer> output, status, control, logits;
     hipEvent_t compute_start = nullptr, compute_end = nullptr;
-    std::unique_ptr<PinnedBuffer> logits, kv, blocks, ffn, scratch;
+    std::unique_ptr<PinnedBuffer> kv, blocks, ffn, scratch;
     std::vector<uint32_t> launch_epochs;  // generation: the exchange epoch of each launch, in order
     bool settled = false;                 // generation: the context's epoch has followed its stop
     std::vector<hipEvent_t> round_events;  // LM-head step: start and end of every round
@@ -207,6 +268,7 @@ struct Context {
     bool matrix_prefill = true;
     std::unique_ptr<MatrixPrefill> matrix;
     size_t instruction_count = 0;
+    std::shared_ptr<PinnedPool> pinned = std::make_shared<PinnedPool>();
     PinnedBuffer ring;
     size_t ring_cursor = 0;
     uint32_t epoch = 1;
@@ -443,10 +505,10 @@ struct Context {
     void finish_ticket(const std::shared_ptr<Ticket>& t, ti_diagnostic_request request)
     {
         const auto& p = model->meta;
-        t->control = std::make_unique<PinnedBuffer>(sizeof(uint64_t));
+        t->control = std::make_unique<PooledBuffer>(pinned, sizeof(uint64_t));
         check(hipMemcpyAsync(t->control->ptr, exchange.ptr, sizeof(uint64_t), hipMemcpyDeviceToHost, stream), "copy control word");
         if (request.logits) {
-            t->logits = std::make_unique<PinnedBuffer>(static_cast<size_t>(std::max(1, p.stack.vocab_size)) * sizeof(float));
+            t->logits = std::make_unique<PooledBuffer>(pinned, static_cast<size_t>(std::max(1, p.stack.vocab_size)) * sizeof(float));
             check(hipMemcpyAsync(t->logits->ptr, logits.ptr, t->logits->bytes, hipMemcpyDeviceToHost, stream), "copy logits");
         }
         if (request.kv) {
@@ -544,8 +606,8 @@ struct Context {
         t->start_position = queued_position;
         t->requested = max_new;
         try {
-            t->output = std::make_unique<PinnedBuffer>(static_cast<size_t>(max_new) * sizeof(ti_token_id));
-            t->status = std::make_unique<PinnedBuffer>(TI_STATUS_WORDS * sizeof(int32_t));
+            t->output = std::make_unique<PooledBuffer>(pinned, static_cast<size_t>(max_new) * sizeof(ti_token_id));
+            t->status = std::make_unique<PooledBuffer>(pinned, TI_STATUS_WORDS * sizeof(int32_t));
             check(hipEventCreate(&t->compute_start), "timing event");
             check(hipEventCreate(&t->compute_end), "timing event");
             check(hipMemsetAsync(status.ptr, 0, status.bytes, stream), "reset selection state");
@@ -594,7 +656,7 @@ struct Context {
             t->hidden = std::make_unique<PinnedBuffer>(bytes);
             std::memcpy(t->hidden->ptr, hidden, bytes);
             check(hipMemcpyAsync(head_hidden.ptr, t->hidden->ptr, bytes, hipMemcpyHostToDevice, stream), "copy hidden vector");
-            t->output = std::make_unique<PinnedBuffer>(sizeof(ti_token_id));
+            t->output = std::make_unique<PooledBuffer>(pinned, sizeof(ti_token_id));
             for (int r = 0; r < rounds; ++r) {
                 hipEvent_t start = nullptr, end = nullptr;
                 check(hipEventCreate(&start), "timing event");

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+from array import array
 from dataclasses import dataclass
 from pathlib import Path
 
@@ -187,6 +188,17 @@ def library() -> C.CDLL:
     return _lib
 
 
+def _token_array(token_ids):
+    """The ids as a C array.  A list or tuple of ints converts as a whole (30,011 ids: 0.2 ms); other
+    sequences, and ids that are not plain 32-bit ints, one by one (1.6 ms) as int() and c_int32 take them."""
+    if isinstance(token_ids, (list, tuple)):
+        try:
+            return (token_id * len(token_ids)).from_buffer(array("i", token_ids))
+        except (TypeError, OverflowError, ValueError):
+            pass
+    return (token_id * len(token_ids))(*[int(t) for t in token_ids])
+
+
 def _check(code: int) -> None:
     if code != 0:
         message = library().ti_last_error_message().decode()
@@ -257,13 +269,46 @@ class Result:
 
 
 class Ticket:
-    def __init__(self, context: "SequenceContext", handle: C.c_void_p, kind: str, requested: int = 0):
-        self._context, self._handle, self.kind, self.requested = context, handle, kind, requested
+    def __init__(self, context: "SequenceContext", handle: C.c_void_p, kind: str, requested: int = 0, kv: bool = False):
+        self._context, self._handle, self.kind, self.requested, self.kv = context, handle, kind, requested, bool(kv)
 
     def __del__(self):
         if getattr(self, "_handle", None) and _lib is not None:
             _lib.ti_ticket_free(self._handle)
             self._handle = None
+
+
+class _Diagnostics(dict):
+    """collect()'s arrays by name.  The K/V array of a request that did not ask for it is zeros, made
+    when it is looked at: it has the whole cache's size, and mapping and unmapping that much memory in
+    a process with a GPU context takes 0.2-0.4 ms."""
+
+    def __init__(self, logits, kv_size, kv, block_outputs):
+        self._kv_size = kv_size
+        super().__init__(logits=logits, kv=kv, block_outputs=block_outputs)
+
+    def _fill(self):
+        if dict.get(self, "kv", 0) is None:
+            self["kv"] = np.zeros(self._kv_size, dtype=np.float32)
+        return self
+
+    def __getitem__(self, name):
+        return dict.__getitem__(self._fill() if name == "kv" else self, name)
+
+    def get(self, name, default=None):
+        return dict.get(self._fill() if name == "kv" else self, name, default)
+
+    def __iter__(self):
+        return dict.__iter__(self._fill())
+
+
+def _filled(name):
+    return lambda self, *args, **kwargs: getattr(dict, name)(self._fill(), *args, **kwargs)
+
+
+for _name in ("keys", "values", "items", "pop", "popitem", "copy", "setdefault", "update", "__eq__", "__ne__", "__or__", "__ror__",
+              "__ior__", "__repr__", "__reversed__", "__reduce_ex__"):
+    setattr(_Diagnostics, _name, _filled(_name))
 
 
 class DecoderModel:
@@ -312,24 +357,24 @@ class SequenceContext:
         return DiagnosticRequest(int(logits), int(kv), int(block_outputs))
 
     def enqueue_prefill(self, token_ids, logits=False, kv=False, block_outputs=False) -> Ticket:
-        ids = (token_id * len(token_ids))(*[int(t) for t in token_ids])
+        ids = _token_array(token_ids)
         handle = C.c_void_p()
         _check(library().ti_context_prefill(self._handle, ids, len(token_ids),
                                             self._request(logits, kv, block_outputs), C.byref(handle)))
-        return Ticket(self, handle, "prefill")
+        return Ticket(self, handle, "prefill", kv=kv)
 
     def enqueue_decode(self, token: int, logits=False, kv=False, block_outputs=False) -> Ticket:
         handle = C.c_void_p()
         _check(library().ti_context_decode(self._handle, int(token), self._request(logits, kv, block_outputs),
                                            C.byref(handle)))
-        return Ticket(self, handle, "prefill")
+        return Ticket(self, handle, "prefill", kv=kv)
 
     def enqueue_generate(self, max_new_tokens: int, eos_id: int | None = None, logits=False, kv=False,
                          block_outputs=False) -> Ticket:
         handle = C.c_void_p()
         _check(library().ti_context_generate(self._handle, int(max_new_tokens), -1 if eos_id is None else int(eos_id),
                                              self._request(logits, kv, block_outputs), C.byref(handle)))
-        return Ticket(self, handle, "generate", max(0, int(max_new_tokens)))
+        return Ticket(self, handle, "generate", max(0, int(max_new_tokens)), kv=kv)
 
     def enqueue_reset(self) -> Ticket:
         handle = C.c_void_p()
@@ -384,12 +429,12 @@ class SequenceContext:
 
     def collect(self, ticket: Ticket) -> dict:
         logits = np.zeros(self.logits_size, dtype=np.float32)
-        kv = np.zeros(self.kv_size, dtype=np.float32)
+        kv = np.zeros(self.kv_size, dtype=np.float32) if ticket.kv else None
         blocks = np.zeros(self.blocks_size, dtype=np.float32)
         fp = C.POINTER(C.c_float)
         _check(library().ti_context_collect(self._handle, ticket._handle, logits.ctypes.data_as(fp),
-                                            kv.ctypes.data_as(fp), blocks.ctypes.data_as(fp)))
-        return {"logits": logits, "kv": kv, "block_outputs": blocks}
+                                            kv.ctypes.data_as(fp) if ticket.kv else None, blocks.ctypes.data_as(fp)))
+        return _Diagnostics(logits, self.kv_size, kv, blocks)
 
     def collect_intermediates(self, ticket: Ticket) -> dict:
         """Scratch vectors (widened, in plan.json's storage.scratch layout) and each layer's FFN
