@@ -10,6 +10,7 @@ sqrt(8) 2^-9 = 0.0055.  A wrong tile, row or part of a sum moves the rows by the
 
 import numpy as np
 import pytest
+import torch
 
 from oracle import decoder as ref
 from tests.test_gpu_prefill import bf16_ulps, kv_rows, oracle_kv_and_logits
@@ -98,3 +99,29 @@ def test_prompt_in_many_parts_then_generation(tmp_path):
         off = float(np.sqrt(((got - expected) ** 2).mean() / (expected ** 2).mean()))
         print(f"off by {off:.5f} of the RMS", flush=True)
         assert off <= 2.0 ** -6
+
+
+def test_short_prompts_hold_small_buffers(tmp_path):
+    """A context of prompts up to 64 tokens holds buffers for 64 rows (here 1.6 MB; the bar leaves room
+    for the allocator's granularity, the long ones take 64 MiB and more), and its rows and logits are
+    bit-equal to those of a context that has taken the long ones."""
+    dims = dict(hidden_size=256, intermediate_size=512, num_attention_heads=4, num_key_value_heads=1, head_dim=64, max_context=160)
+    spec = P.StackSpec(P.BlockSpec(**dims), 2, 512, True)
+    K.build_stack_package(spec, K.random_weights(spec, seed=3, std=0.08), probe.probe_library(), tmp_path / "pkg", "bfloat16")
+    model = R.DecoderModel(R.load_plan(tmp_path / "pkg"))
+    fresh, used = model.create_context(), model.create_context()
+    prompt = np.random.default_rng(1).integers(0, 512, 64).tolist()
+    used.wait(used.enqueue_prefill(prompt + prompt[:40]))
+    used.wait(used.enqueue_reset())
+    fresh.wait(fresh.enqueue_decode(1))  # the code of a first launch is loaded
+    fresh.wait(fresh.enqueue_reset())
+    free = torch.cuda.mem_get_info()[0]
+    got = fresh.collect(fresh.enqueue_prefill(prompt, logits=True, kv=True))
+    held = free - torch.cuda.mem_get_info()[0]
+    want = used.collect(used.enqueue_prefill(prompt, logits=True, kv=True))
+    assert held <= 16 << 20, held
+    assert np.array_equal(got["kv"], want["kv"]) and np.array_equal(got["logits"], want["logits"])
+    for ctx in (fresh, used):
+        ctx.wait(ctx.enqueue_reset())
+    got, want = (c.collect(c.enqueue_prefill(prompt + prompt[:40], logits=True))["logits"] for c in (fresh, used))
+    assert np.array_equal(got, want)

@@ -480,7 +480,7 @@ struct TileShape {
 constexpr TileShape kTileShapes[] = {{256, 256, 2.03f, 0.0f}, {128, 128, 0.85f, 1.1f}, {128, 64, 0.52f, 0.74f}, {64, 64, 0.29f, 0.46f}};
 constexpr float kBlockStart = 2.4f;         // us a block takes besides its K steps
 constexpr float kPartialRate = 3.1e6f;      // bytes per us that partial sums are written and read back at
-constexpr size_t kPartialFloats = 16u << 20;  // 64 MiB of partial sums
+constexpr size_t kPartialFloats = 16u << 20;  // 64 MiB of partial sums at most
 
 struct Tiling {
     int shape, splits;
@@ -559,8 +559,9 @@ MatrixPrefill::MatrixPrefill(const ti_worker_program_view& program) : p_(program
 
 MatrixPrefill::~MatrixPrefill()
 {
-    if (buffer_)
-        (void)hipFree(buffer_);
+    for (const Buffer& b : {short_, long_})
+        if (b.data)
+            (void)hipFree(b.data);
 }
 
 namespace {
@@ -575,12 +576,18 @@ size_t row_elements(const ti_model_shape& s)
     const size_t q = static_cast<size_t>(s.query_heads) * s.head_dim;
     return 3 * d + qkv + 2 * q + f;  // x, u, r | qkv | q, attention | product
 }
+// The partial sums of any product of `rows` rows that choose_tiling splits.
+size_t partial_elements(const ti_model_shape& s, size_t rows)
+{
+    const size_t widest = std::max<size_t>(s.hidden_size, static_cast<size_t>(s.query_heads + 2 * s.kv_heads) * s.head_dim);
+    return std::min(kPartialFloats, kMostSplits * rows * widest);
+}
 Views views(void* buffer, const ti_model_shape& s, size_t rows)
 {
     const size_t d = s.hidden_size, q = static_cast<size_t>(s.query_heads) * s.head_dim;
     Views v{};
     v.partial = static_cast<float*>(buffer);
-    uint16_t* at = reinterpret_cast<uint16_t*>(v.partial + kPartialFloats);
+    uint16_t* at = reinterpret_cast<uint16_t*>(v.partial + partial_elements(s, rows));
     auto take = [&](size_t per_row) {
         uint16_t* start = at;
         at += rows * per_row;
@@ -685,7 +692,7 @@ void MatrixPrefill::feed_forward(hipStream_t stream, int layer, int rows, int fi
     const int d = s.hidden_size, f = s.intermediate_size, qw = s.query_heads * s.head_dim;
     const ti_layer_layout& w = p_.layout;
     const uint16_t* base = weights(layer);
-    const Views v = views(buffer_, s, kChunkRows);
+    const Views v = views(buffer_.data, s, buffer_.rows);
     uint16_t* x = v.x + static_cast<size_t>(first_row) * d;
     const float eps = p_.numeric.rms_norm_eps;
     const GemmRows projected = gemm(stream, v.attention, rows, qw, base + w.Wo, d, x, v.r, d, v.partial);
@@ -702,7 +709,7 @@ int MatrixPrefill::layer(hipStream_t stream, void* kv, int layer, int position, 
     const ti_model_shape& s = p_.shape;
     const int d = s.hidden_size, dh = s.head_dim, nq = s.query_heads, nkv = s.kv_heads;
     const int qw = nq * dh, kvw = nkv * dh;
-    const Views v = views(buffer_, s, kChunkRows);
+    const Views v = views(buffer_.data, s, buffer_.rows);
     const ti_layer_layout& w = p_.layout;
     const uint16_t* base = weights(layer);
     uint16_t* cache = static_cast<uint16_t*>(kv) + static_cast<size_t>(layer) * p_.stack.layer_kv_stride;
@@ -738,11 +745,11 @@ int MatrixPrefill::layer(hipStream_t stream, void* kv, int layer, int position, 
 
 int MatrixPrefill::last_row(hipStream_t stream, void* kv, int position, const void** hidden)
 {
-    if (!buffer_ || rows_ < 1 || position < rows_ - 1)
+    if (!buffer_.data || rows_ < 1 || position < rows_ - 1)
         return fail(TI_ERR_INVALID_ARGUMENT, "no prefilled position to finish");
     const ti_model_shape& s = p_.shape;
     const int d = s.hidden_size, dh = s.head_dim, nq = s.query_heads, nkv = s.kv_heads, layer = p_.stack.layers - 1;
-    const Views v = views(buffer_, s, kChunkRows);
+    const Views v = views(buffer_.data, s, buffer_.rows);
     const ti_layer_layout& w = p_.layout;
     const uint16_t* cache = static_cast<const uint16_t*>(kv) + static_cast<size_t>(layer) * p_.stack.layer_kv_stride;
     const size_t row = rows_ - 1;
@@ -756,6 +763,26 @@ int MatrixPrefill::last_row(hipStream_t stream, void* kv, int position, const vo
     return e == hipSuccess ? TI_OK : hip_fail(e, "prefill kernel launch");
 }
 
+int MatrixPrefill::reserve(int count)
+{
+    if (long_.data || (short_.data && count <= kShortRows)) {
+        buffer_ = long_.data ? long_ : short_;
+        return TI_OK;
+    }
+    Buffer& b = count <= kShortRows ? short_ : long_;
+    const int rows = count <= kShortRows ? kShortRows : kChunkRows;
+    const size_t bytes = partial_elements(p_.shape, rows) * sizeof(float) + row_elements(p_.shape) * rows * sizeof(uint16_t);
+    const hipError_t e = hipMalloc(&b.data, bytes);
+    if (e != hipSuccess) {
+        b.data = nullptr;
+        (void)hipGetLastError();  // the caller may go on without: the next launch's check is not to see it
+        return hip_fail(e, "prefill buffers");
+    }
+    b.rows = rows;
+    buffer_ = b;
+    return TI_OK;
+}
+
 int MatrixPrefill::enqueue(hipStream_t stream, void* kv, const ti_token_id* tokens, int position, int count)
 {
     if (!supports(p_))
@@ -764,15 +791,10 @@ int MatrixPrefill::enqueue(hipStream_t stream, void* kv, const ti_token_id* toke
         return TI_OK;
     if (position < 0 || position + count > p_.shape.max_context)
         return fail(TI_ERR_INVALID_ARGUMENT, "sequence context capacity reached");
-    if (!buffer_) {
-        buffer_bytes_ = kPartialFloats * sizeof(float) + row_elements(p_.shape) * kChunkRows * sizeof(uint16_t);
-        const hipError_t e = hipMalloc(&buffer_, buffer_bytes_);
-        if (e != hipSuccess) {
-            buffer_ = nullptr;
-            return hip_fail(e, "prefill buffers");
-        }
-    }
-    const Views v = views(buffer_, p_.shape, kChunkRows);
+    const int code = reserve(count);
+    if (code != TI_OK)
+        return code;
+    const Views v = views(buffer_.data, p_.shape, buffer_.rows);
     const uint16_t* embedding = static_cast<const uint16_t*>(p_.weights) + p_.stack.embedding_offset;
     for (int first = 0; first < count; first += kChunkRows) {
         const int rows = rows_ = std::min(kChunkRows, count - first);

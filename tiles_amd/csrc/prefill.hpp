@@ -15,6 +15,9 @@ class MatrixPrefill {
   public:
     // Positions per pass through the layers: the activation buffers hold this many rows.
     static constexpr int kChunkRows = 4096;
+    // Or this many, for an object that has seen no longer prompt: 9 MB at Llama-3.2-1B widths instead of
+    // 243, so that many contexts with short prompts hold little each.
+    static constexpr int kShortRows = TI_MAX_LAUNCH_STEPS;
     // The shortest prompt that takes this path: its kernels read every weight once, in about the time of
     // two worker steps (Llama-3.2-1B: 3 tokens 1.34 ms against 1.97 through the worker, 37 tokens 1.45
     // against 19.2, 2 tokens 1.39 against 1.45; two of its layers alone: 3 tokens 0.68 against 0.77).
@@ -33,6 +36,9 @@ class MatrixPrefill {
     // Whether a package of this kind can be prefilled with matrices (bf16 decoder stacks).
     static bool supports(const ti_worker_program_view& program);
 
+    // Makes sure of buffers for `count` positions, which enqueue() otherwise does itself.  On failure
+    // (TI_* code, no memory) the object is as before.
+    int reserve(int count);
     // Enqueues positions [position, position + count) of the prompt whose token ids are at
     // `tokens` (device memory, `count` of them) on `stream`: every layer's K and V rows of those
     // positions go into `kv`.  The positions before `position` must already be in the cache.
@@ -44,8 +50,12 @@ class MatrixPrefill {
 
   private:
     ti_worker_program_view p_;
-    void* buffer_ = nullptr;  // every activation buffer, kChunkRows rows each
-    size_t buffer_bytes_ = 0;
+    struct Buffer {
+        void* data = nullptr;  // the partial sums and every activation buffer
+        int rows = 0;          // of each
+    };
+    Buffer short_, long_;  // kept; a short one too when a long one follows, as queued work may use it
+    Buffer buffer_;        // the one in use
     int rows_ = 0;  // of the last pass: positions it left in the activation buffers
     int layer(hipStream_t stream, void* kv, int layer, int position, int rows);
     const uint16_t* weights(int layer) const;

@@ -115,7 +115,8 @@ __device__ inline void gemm_store(const GemmArgs& g, int m0, int n0, int split, 
 // chunks of a row are exchanged at the source: chunk c of staged row r lies at c ^ r mod 8 (KS 64), so
 // that the 16 rows of an operand read fall on distinct banks (no bank conflicts counted).
 // Rows past m and n are clamped on load and not stored.  k % KS == 0, n % 8 == 0, ldc % 8 == 0 and
-// 16-byte aligned pointers (the launcher checks).
+// 16-byte aligned pointers (MatrixPrefill::supports
+// holds widths to multiples of 16, so every row starts aligned).
 template <int BM, int BN, int WM, int WN, int KS, int STAGES, GemmOut OUT>
 __global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64) gemm_tiles(GemmArgs g)
 {

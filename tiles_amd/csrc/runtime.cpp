@@ -543,6 +543,20 @@ struct Context {
         outstanding.push_back(t);
     }
 
+    // Whether a prompt of n tokens goes through the matrices; their buffers are there then.  Without
+    // memory for them, a prompt of one launch goes through the worker, which needs none.
+    bool prefills_with_matrices(int n)
+    {
+        if (!matrix_prefill || n < MatrixPrefill::kMinPrompt || !MatrixPrefill::supports(model->view))
+            return false;
+        if (!matrix)
+            matrix = std::make_unique<MatrixPrefill>(model->view);
+        const int code = matrix->reserve(n);
+        if (code != TI_OK && n > TI_MAX_LAUNCH_STEPS)
+            check_ti(code);
+        return code == TI_OK;
+    }
+
     std::shared_ptr<Ticket> prefill(const ti_token_id* ids, size_t count, ti_diagnostic_request diag)
     {
         require_ready();
@@ -561,9 +575,7 @@ struct Context {
         try {
             stage_input(ids, count);
             const int n = static_cast<int>(count);
-            if (matrix_prefill && n >= MatrixPrefill::kMinPrompt && MatrixPrefill::supports(model->view)) {
-                if (!matrix)
-                    matrix = std::make_unique<MatrixPrefill>(model->view);
+            if (prefills_with_matrices(n)) {
                 // The last token leaves the logits and greedy candidates that a generation or collect()
                 // continues from: through the matrices and the logits tasks, or, where its position
                 // is far, or the diagnostics or the timeline of a whole step are asked for, through a
